@@ -274,10 +274,10 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     uint64_t floats = 0;
     for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
       if (r == 0) continue;
-      const uint32_t sp = qi::gemm_split_splits(im, r);
+      const uint32_t sp = qi::gemm_split_splits(im, r, chunk, kScratchBytes);
       if (sp > 1) floats = std::max(floats, static_cast<uint64_t>(sp) * r * im.n);
     }
-    p->splits = qi::gemm_split_splits(im, chunk);
+    p->splits = qi::gemm_split_splits(im, chunk, chunk, kScratchBytes);
     p->s_floats = floats;
     p->d_floats = (qi::gemm_split_records_bytes(chunk, im.k) + 3) / 4;
     return QI_HIP_OK;
@@ -398,8 +398,9 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
     case LinearPlan::kSplitGemm:
       for (uint64_t m0 = 0; m0 < m; m0 += kSplitChunkRows) {
         const uint64_t rows = m - m0 < kSplitChunkRows ? m - m0 : kSplitChunkRows;
-        QI_HIP_TRY(qi::launch_gemm_split(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws,
-                                         qi::gemm_split_splits(im, rows), reinterpret_cast<uint8_t*>(dws), st),
+        const uint32_t sp = qi::gemm_split_splits(im, rows, m < kSplitChunkRows ? m : kSplitChunkRows, kScratchBytes);
+        QI_HIP_TRY(qi::launch_gemm_split(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, sp,
+                                         reinterpret_cast<uint8_t*>(dws), st),
                    "launch split-half gemm");
       }
       return QI_HIP_OK;

@@ -90,7 +90,10 @@ hipError_t launch_gemv_half(int32_t qtype, bool wide, const View& w, const float
 // added in order.
 bool gemm_split_supported(const Image& im);
 uint64_t gemm_split_records_bytes(uint64_t m, uint64_t k);
-uint32_t gemm_split_splits(const Image& im, uint64_t m);
+// K parts of m rows of a call whose records hold `records_rows` rows (its
+// longest chunk): partial sums and records together within `scratch_bytes`,
+// or one part.
+uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t records_rows, uint64_t scratch_bytes);
 hipError_t launch_gemm_split(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
                              uint32_t splits, uint8_t* records, hipStream_t st);
 

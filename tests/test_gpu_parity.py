@@ -391,6 +391,21 @@ def test_f32_split_gemm_tolerance(ctx, qtype, shape):
     w.free()
 
 
+@pytest.mark.parametrize("qtype", [qa.Q4_K, qa.Q6_K], ids=lambda q: NAMES[q])
+@pytest.mark.parametrize("k,n,m", [(2816, 1040, 34), (2816, 1040, 130), (12288, 2048, 70), (3328, 8208, 200)])
+def test_f32_split_gemm_part_counts(ctx, qtype, k, n, m):
+    """K parts of one unit (11 units in 11 parts), parts of several units and
+    uneven ones, a ragged last tile: the F32 bars (1e-5, as for every f32 sum
+    of exact products here)."""
+    blocks = po.make_weights(qtype, k, n, seed=4980 + qtype + k, outliers=True)
+    w = ctx.weights(qtype, qa.OUTPUT_ROWS, k, n, blocks)
+    x = po.fill_normal(4990 + m, m * k).reshape(m, k)
+    y = w.linear(x, qa.MODE_F32)
+    _assert_f32(y, x, blocks, qtype, n, (k, n, m))
+    assert w.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+    w.free()
+
+
 def test_f32_split_gemm_row_chunks(ctx):
     """Calls above 4096 rows run in 4096-row launches (bounded activation
     records): 4156 rows equal the 4096-row and 60-row calls of the same rows
