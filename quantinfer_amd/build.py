@@ -54,7 +54,8 @@ FLAGS = [
 # default: their 128-register accumulator tiles need the accumulator file.
 FILE_FLAGS = {"qi_gemv_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "qi_gemv_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-              "qi_gemv_rm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+              "qi_gemv_rm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "qi_gemm_bf3.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def hipcc() -> str:

@@ -170,10 +170,11 @@ qi_hip_status grow_ws(qi_hip_ctx* c, hipStream_t st, float** buf, uint64_t* cap,
 // function decides, so that the growing path (run_linear) and the scratch
 // path (qi_hip_linear_device_noalloc) take the same kernels.
 struct LinearPlan {
-  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kF32Gemm, kExact } kind = kExact;
+  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kBf3Gemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kExact } kind = kExact;
   uint64_t m_pad = 0;
   uint32_t splits = 1;  // GEMM K splits, or row-major GEMV K splits per row chunk
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
+  uint64_t part_floats = 0;  // kBf3Gemm, kSplitGemm: the most that partial sums may take
 };
 
 // Rows from which row-major weights (tiled image, K a multiple of 4) take
@@ -188,6 +189,11 @@ struct LinearPlan {
 constexpr uint64_t kRmGemmMinRows = 3;
 constexpr uint64_t kRmGemmChunkRows = 4096;
 constexpr uint64_t kRmPartFloats = 8ull << 20;
+
+// F32 weights' GEMM (qi_gemm_bf3.hip): calls run in chunks of kBf3ChunkRows
+// rows; the K parts' partial sums take at most kBf3PartFloats.
+constexpr uint64_t kBf3ChunkRows = 4096;
+constexpr uint64_t kBf3PartFloats = 8ull << 20;
 
 // Rows of a chunk at which the 2-16 row GEMV switches from the int8-digit
 // kernel (qi_gemv_rows.hip) to the split-half kernel (qi_gemv_half.hip): the
@@ -210,6 +216,21 @@ constexpr uint64_t kSplitMinRows = 33;
 // Rows per split-half GEMM launch: longer calls run in chunks, so that the
 // activation records (about 4.1 bytes per activation) stay bounded.
 constexpr uint64_t kSplitChunkRows = 4096;
+
+// K parts of F32 weights' GEMM and of the split-half GEMM, their partial sums
+// within p->part_floats. Calls run in chunks; a shorter last chunk takes its
+// own part count (enqueue_linear asks again).
+void plan_parts(const Image& im, uint64_t m, LinearPlan* p) {
+  const bool bf3 = p->kind == LinearPlan::kBf3Gemm;
+  const uint64_t rows = bf3 ? kBf3ChunkRows : kSplitChunkRows, chunk = m < rows ? m : rows;
+  p->s_floats = 0;
+  for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
+    if (r == 0) continue;
+    const uint32_t parts = bf3 ? qi::gemm_bf3_plan(im, r, p->part_floats).parts
+                               : qi::gemm_split_splits(im, r, p->part_floats);
+    if (parts > 1) p->s_floats = std::max(p->s_floats, static_cast<uint64_t>(parts) * r * im.n);
+  }
+}
 
 qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan* p) {
   if (mode < QI_HIP_MODE_AUTO || mode > QI_HIP_MODE_MFMA)
@@ -236,8 +257,10 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
   }
   if (mode != QI_HIP_MODE_EXACT && qi::f32w_gemv_supported(im)) {
     // F32 weights: the streaming GEMV in 8-row chunks, the matrix-core GEMM above
-    if (m > qi::kF32GemvMaxRows && qi::f32w_gemm_supported(im)) {
-      p->kind = LinearPlan::kF32Gemm;
+    if (m > qi::kF32GemvMaxRows && qi::gemm_bf3_supported(im)) {
+      p->kind = LinearPlan::kBf3Gemm;
+      p->part_floats = kBf3PartFloats;
+      plan_parts(im, m, p);
       return QI_HIP_OK;
     }
     p->kind = LinearPlan::kF32Gemv;
@@ -268,18 +291,13 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
   }
   if (mode != QI_HIP_MODE_EXACT && m >= kSplitMinRows && qi::gemm_split_supported(im)) {
     p->kind = LinearPlan::kSplitGemm;
-    // chunks of kSplitChunkRows rows; a shorter last chunk takes its own K
-    // split count (enqueue_linear asks again)
+    // partial sums beside the records of a chunk within the no-allocation
+    // entry point's scratch where both fit
     const uint64_t chunk = m < kSplitChunkRows ? m : kSplitChunkRows;
-    uint64_t floats = 0;
-    for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
-      if (r == 0) continue;
-      const uint32_t sp = qi::gemm_split_splits(im, r, chunk, kScratchBytes);
-      if (sp > 1) floats = std::max(floats, static_cast<uint64_t>(sp) * r * im.n);
-    }
-    p->splits = qi::gemm_split_splits(im, chunk, chunk, kScratchBytes);
-    p->s_floats = floats;
-    p->d_floats = (qi::gemm_split_records_bytes(chunk, im.k) + 3) / 4;
+    const uint64_t records = qi::gemm_split_records_bytes(chunk, im.k);
+    p->d_floats = (records + 3) / 4;
+    p->part_floats = (records < kScratchBytes ? kScratchBytes - records : kScratchBytes) / 4;
+    plan_parts(im, m, p);
     return QI_HIP_OK;
   }
   if (mode != QI_HIP_MODE_EXACT && qi::gemv_mfma_supported(im.qtype, im.layout, im.k)) {
@@ -353,6 +371,14 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
                    "launch row-major GEMM");
       }
       return QI_HIP_OK;
+    case LinearPlan::kBf3Gemm:
+      for (uint64_t m0 = 0; m0 < m; m0 += kBf3ChunkRows) {
+        const uint64_t rows = m - m0 < kBf3ChunkRows ? m - m0 : kBf3ChunkRows;
+        QI_HIP_TRY(qi::launch_gemm_bf3(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws,
+                                       qi::gemm_bf3_plan(im, rows, p.part_floats), st),
+                   "launch f32 GEMM");
+      }
+      return QI_HIP_OK;
     case LinearPlan::kMfma:
     case LinearPlan::kPlanar:
       for (uint64_t m0 = 0; m0 < m; m0 += 16) {
@@ -398,7 +424,7 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
     case LinearPlan::kSplitGemm:
       for (uint64_t m0 = 0; m0 < m; m0 += kSplitChunkRows) {
         const uint64_t rows = m - m0 < kSplitChunkRows ? m - m0 : kSplitChunkRows;
-        const uint32_t sp = qi::gemm_split_splits(im, rows, m < kSplitChunkRows ? m : kSplitChunkRows, kScratchBytes);
+        const uint32_t sp = qi::gemm_split_splits(im, rows, p.part_floats);
         QI_HIP_TRY(qi::launch_gemm_split(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, sp,
                                          reinterpret_cast<uint8_t*>(dws), st),
                    "launch split-half gemm");
@@ -410,9 +436,6 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
         QI_HIP_TRY(qi::launch_f32w_gemv(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, p.splits, st),
                    "launch f32 gemv");
       }
-      return QI_HIP_OK;
-    case LinearPlan::kF32Gemm:
-      QI_HIP_TRY(qi::launch_f32w_gemm(im, v, x, m, y, st), "launch f32 gemm");
       return QI_HIP_OK;
     case LinearPlan::kExact:
       QI_HIP_TRY(qi::launch_exact(im, v, x, m, y, st), "launch exact matmul");
@@ -427,6 +450,14 @@ qi_hip_status run_linear(qi_hip_ctx* c, const qi_hip_weights* w, const float* x,
   LinearPlan p;
   qi_hip_status s = plan_linear(w->im, m, mode, &p);
   if (s != QI_HIP_OK) return s;
+  // A stream under capture cannot allocate: fewer K parts where the partial
+  // sums' workspace does not hold them all yet. F32 weights' GEMM, which
+  // needs nothing else from the context, then uses no workspace at all.
+  const bool bf3 = p.kind == LinearPlan::kBf3Gemm;
+  if (p.s_floats > 0 && (bf3 || (p.kind == LinearPlan::kSplitGemm && p.s_floats > c->scap)) && capturing(st)) {
+    p.part_floats = bf3 ? 0 : c->scap;
+    plan_parts(w->im, m, &p);
+  }
   if ((s = grow_ws(c, st, &c->hbuf, &c->hcap, p.h_floats, "alloc GEMM workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->sbuf, &c->scap, p.s_floats, "alloc split-K workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->dbuf, &c->dcap, p.d_floats, "alloc GEMV workspace")) != QI_HIP_OK) return s;

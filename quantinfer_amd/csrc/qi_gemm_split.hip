@@ -286,14 +286,13 @@ uint64_t gemm_split_records_bytes(uint64_t m, uint64_t k) {
   return (m + kSRows - 1) / kSRows * (k / 256) * kSStage;
 }
 
-uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t records_rows, uint64_t scratch_bytes) {
+uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t part_floats) {
   // One workgroup per CU, so a launch takes whole rounds of 256 blocks, and a
   // last round that is nearly empty costs as much as a full one: 336 blocks
   // (Q6_K 333 x 4096 x 14336) took two rounds of 16 units. Of the counts whose
-  // partial sums fit beside the records in `scratch_bytes`, the one with the
-  // least modelled time: rounds x units of a part x the time of a unit, the
-  // sum launch, and the partial sums' trip through memory. The constants are
-  // fits to counts 1 to 16 at 11 shapes (MI355X; model within 10%). Against
+  // partial sums fit in `part_floats`, the one with the least modelled time:
+  // rounds x units of a part x the time of a unit, the sum launch, and the
+  // partial sums' trip through memory. The constants are fits to counts 1 to 16 at 11 shapes (MI355X; model within 10%). Against
   // the rule before (fill 256 CUs once, rounded up, at least 4 units a part),
   // us per call: Q4_K M=300 12288 x 4096 136.7 -> 95.4 (80 blocks: 3 parts for
   // 4), 4096 x 6144 82.2 -> 61.4 (2 for 3), 4096 x 4096 63.3 -> 51.3; Q6_K
@@ -303,13 +302,12 @@ uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t records_rows, u
   constexpr double kSumUs = 3.0, kPartUsPerByte = 0.37e-6;
   const uint64_t gt = split_group_tiles();
   const uint64_t blocks = (m + kSRows - 1) / kSRows * ((im.tiles + gt - 1) / gt);
-  const uint64_t units = im.k / 256, records = gemm_split_records_bytes(records_rows, im.k);
-  const uint64_t room = records < scratch_bytes ? scratch_bytes - records : scratch_bytes;
+  const uint64_t units = im.k / 256;
   uint64_t best = 1;
   double best_us = 0.0;
   for (uint64_t s = 1; s <= units && s <= 32; ++s) {
     const uint64_t part_units = (units + s - 1) / s, bytes = s > 1 ? s * m * im.n * 4 : 0;
-    if (bytes > room) break;
+    if (bytes > 4 * part_floats) break;
     // the same longest part with fewer parts: only the fewest
     if (s > 1 && (units + part_units - 1) / part_units != s) continue;
     const uint64_t rounds = (blocks * s + kSCUs - 1) / kSCUs;

@@ -90,10 +90,8 @@ hipError_t launch_gemv_half(int32_t qtype, bool wide, const View& w, const float
 // added in order.
 bool gemm_split_supported(const Image& im);
 uint64_t gemm_split_records_bytes(uint64_t m, uint64_t k);
-// K parts of m rows of a call whose records hold `records_rows` rows (its
-// longest chunk): partial sums and records together within `scratch_bytes`,
-// or one part.
-uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t records_rows, uint64_t scratch_bytes);
+// K parts of m rows, their partial sums within `part_floats` (or one part).
+uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t part_floats);
 hipError_t launch_gemm_split(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
                              uint32_t splits, uint8_t* records, hipStream_t st);
 
@@ -115,20 +113,36 @@ uint32_t rm_gemm_parts(const Image& im, uint64_t m, uint64_t max_part_floats);
 hipError_t launch_rm_gemm(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
                           uint32_t parts, hipStream_t st);
 
+// y = the sum of `splits` partial results of `count` = m * n values in split
+// order; a non-finite sum is recomputed in the reference's order.
+hipError_t launch_f32w_sum(const View& v, const float* part, uint32_t splits, uint64_t count, float* y,
+                           const float* x, hipStream_t st);
+
+// GEMM of F32 weights (K and N multiples of 4) with f32 accuracy on the bf16
+// matrix cores (qi_gemm_bf3.hip). K is split into plan.parts (the partial sums
+// in `part`, parts * m * n floats, when parts > 1); non-finite outputs are
+// recomputed in the reference's order.
+struct Bf3Plan {
+  uint32_t tm = 0, wm = 0;  // a workgroup's rows: 16 tm wm, by 4 wm wavefronts
+  uint32_t parts = 1;
+};
+bool gemm_bf3_supported(const Image& im);
+Bf3Plan gemm_bf3_plan(const Image& im, uint64_t m, uint64_t max_part_floats);
+hipError_t launch_gemm_bf3(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
+                           const Bf3Plan& plan, hipStream_t st);
+
 // F32 weights (row-major [K, N] f32, N a multiple of 4): the streaming GEMV
 // for up to 8 rows per launch (K split over the grid; `part` holds splits * m * n floats
-// when splits > 1), and the matrix-core GEMM for more rows (K a multiple of
-// 4; no workspace).
-// rows above which F32 weights take the GEMM: at the LM head shape
-// (4096 x 151936) 9-16 rows take 0.55-0.64 ms on the 32-row GEMM tiles
-// against 0.97-1.11 ms for two GEMV launches; 8 rows 0.56 ms on one GEMV
-constexpr uint64_t kF32GemvMaxRows = 8;
+// when splits > 1); more rows take the GEMM above.
+// rows above which F32 weights take the GEMM. us per call, GEMV / GEMM (MI355X):
+// 3 rows 4096 x 4096 28.0 / 26.8, 4096 x 14336 50 / 54; 4 rows 2048 x 8192 28.3 /
+// 23.3, 4096 x 14336 49.6 / 54.5, 4096 x 151936 435 / 444; 8 rows (the GEMV's
+// 8-row launch) 38.1 / 23.7, 60.2 / 49.9, 556 / 460
+constexpr uint64_t kF32GemvMaxRows = 4;
 bool f32w_gemv_supported(const Image& im);
 uint32_t f32w_splits(const Image& im);
 hipError_t launch_f32w_gemv(const Image& im, const View& v, const float* x, uint32_t m, float* y, float* part,
                             uint32_t splits, hipStream_t st);
-bool f32w_gemm_supported(const Image& im);
-hipError_t launch_f32w_gemm(const Image& im, const View& v, const float* x, uint64_t m, float* y, hipStream_t st);
 
 // Exact-order matmul: bit-identical to CpuScalar (any M, either layout).
 hipError_t launch_exact(const Image& im, const View& w, const float* x, uint64_t m, float* y,

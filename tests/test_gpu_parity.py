@@ -792,6 +792,78 @@ def test_f32_weights_gemm_edges(ctx, k, n):
     wt.free()
 
 
+@pytest.mark.parametrize("k,n", [(4, 4), (36, 256), (100, 260), (1028, 516), (3104, 3000)])
+def test_f32_weights_gemm_tiles(ctx, k, n):
+    """The F32 weights' GEMM at the edges of its tiles: one stage of 32 k and
+    less, a partial last stage, columns past a 256-column tile, row counts at
+    and past every tile height (16 to 128), K parts and none. Bars of 1e-5 as
+    for every F32-mode sum; the 2-norm error stays below 3e-7 (three times what
+    exact products and f32 sums of 97 additions leave at K = 3104)."""
+    w = po.fill_normal(9840 + k, k * n, 0.02).reshape(k, n)
+    wt = ctx.weights(qa.F32, qa.ROW_MAJOR, k, n, w)
+    for m in (5, 16, 17, 33, 49, 64, 65, 97, 130, 300):
+        x = po.fill_normal(9841 + m, m * k).reshape(m, k)
+        y = wt.linear(x, qa.MODE_F32)
+        comp, norm = _f32w_checks(y, x, w)
+        e = x.astype(np.float64) @ w.astype(np.float64)
+        rel = np.linalg.norm(y - e) / np.linalg.norm(e)
+        assert comp <= F32_TOL and norm <= F32_TOL and rel <= 3e-7, (k, n, m, comp, norm, rel)
+        assert wt.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+    wt.free()
+
+
+def test_f32_weights_gemm_pieces_are_exact(ctx):
+    """Every f32 weight is the sum of its three bf16 pieces: with one-hot
+    activation rows the outputs are weight rows bit for bit, over magnitudes
+    from 2^-100 to 2^100."""
+    k, n, m = 260, 512, 70
+    rng = np.random.default_rng(9860)
+    w = (rng.standard_normal((k, n)) * 2.0 ** rng.integers(-100, 101, (k, n))).astype(np.float32)
+    wt = ctx.weights(qa.F32, qa.ROW_MAJOR, k, n, w)
+    picks = rng.integers(0, k, m)
+    x = np.zeros((m, k), np.float32)
+    x[np.arange(m), picks] = 1.0
+    assert np.array_equal(wt.linear(x, qa.MODE_F32), w[picks])
+    wt.free()
+
+
+def test_f32_weights_gemm_under_capture():
+    """A stream under capture allocates nothing: on a fresh context the F32
+    weights' GEMM is captured without K parts, and each replay gives the same
+    outputs, within the F32 bars."""
+    import ctypes
+    from quantinfer_amd import hiprt
+    k, n, m = 2048, 512, 40
+    w = po.fill_normal(9870, k * n, 0.02).reshape(k, n)
+    x = po.fill_normal(9871, m * k).reshape(m, k)
+    with qa.Context(0) as c:
+        wt = c.weights(qa.F32, qa.ROW_MAJOR, k, n, w)
+        xd, yd = hiprt.DeviceBuffer.from_array(x), hiprt.DeviceBuffer(m * n * 4)
+        st, h = hiprt.Stream(), hiprt.hip()
+        graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+        vp = ctypes.c_void_p
+        assert h.hipStreamBeginCapture(vp(st.handle), 1) == 0
+        wt.linear_device(xd.ptr, m, yd.ptr, qa.MODE_F32, st.handle)
+        assert h.hipStreamEndCapture(vp(st.handle), ctypes.byref(graph)) == 0
+        assert h.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+        outs = []
+        for _ in range(3):
+            yd.zero()
+            hiprt.synchronize()
+            assert h.hipGraphLaunch(ex, vp(st.handle)) == 0
+            st.synchronize()
+            outs.append(yd.to_array(np.float32, (m, n)))
+            eager = wt.linear(x, qa.MODE_F32)
+        comp, norm = _f32w_checks(outs[0], x, w)
+        assert comp <= F32_TOL and norm <= F32_TOL
+        assert normwise_rel_err(eager, outs[0]) <= F32_TOL
+        assert all(o.tobytes() == outs[0].tobytes() for o in outs)
+        h.hipGraphExecDestroy(ex)
+        h.hipGraphDestroy(graph)
+        st.destroy()
+        wt.free()
+
+
 def test_f32_weights_lm_head_shape(ctx):
     """The unchanged runtime's LM head: [4096, 151936] f32 (a Q6_K head
     dequantized at load, runtime/src/qwen3/loader.rs:47-61), one decode row
