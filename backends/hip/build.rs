@@ -28,6 +28,7 @@ const FILE_FLAGS: &[(&str, &[&str])] = &[
     ("qi_gemv_rows.hip", &["-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("qi_gemv_rm.hip", &["-mllvm", "-amdgpu-mfma-vgpr-form"]),
     ("qi_gemm_bf3.hip", &["-mllvm", "-amdgpu-mfma-vgpr-form"]),
+    ("qi_gemm_rm.hip", &["-mllvm", "-amdgpu-mfma-vgpr-form"]),
 ];
 
 fn main() {

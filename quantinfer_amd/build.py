@@ -55,7 +55,8 @@ FLAGS = [
 FILE_FLAGS = {"qi_gemv_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "qi_gemv_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "qi_gemv_rm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-              "qi_gemm_bf3.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+              "qi_gemm_bf3.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "qi_gemm_rm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def hipcc() -> str:

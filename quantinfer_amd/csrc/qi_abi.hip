@@ -170,22 +170,24 @@ qi_hip_status grow_ws(qi_hip_ctx* c, hipStream_t st, float** buf, uint64_t* cap,
 // function decides, so that the growing path (run_linear) and the scratch
 // path (qi_hip_linear_device_noalloc) take the same kernels.
 struct LinearPlan {
-  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kBf3Gemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kExact } kind = kExact;
+  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kRmGemm, kBf3Gemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kExact } kind = kExact;
   uint64_t m_pad = 0;
   uint32_t splits = 1;  // GEMM K splits, or row-major GEMV K splits per row chunk
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
   uint64_t part_floats = 0;  // kBf3Gemm, kSplitGemm: the most that partial sums may take
 };
 
-// Rows from which row-major weights (tiled image, K a multiple of 4) take
-// the row-major GEMM (weights dequantized into LDS for the f32 matrix cores,
-// K split into parts whose partial sums take at most kRmPartFloats) instead
-// of the GEMV's 2-row launches, each of which reads and converts the whole
-// weight. Calls run in chunks of kRmGemmChunkRows rows. Measured on MI355X,
-// us per call, Q4_K 4096x14336, GEMV launches / GEMM: M=2 28.0 / 36.4,
-// M=4 54.7 / 37.7, M=16 211.6 / 39.6, M=64 838 / 105 (the K-slice GEMM it
-// replaced, f32 weight slices dequantized to HBM: 580), M=512 843 (K slices)
-// / 660, M=2048 2446 (K slices) / 2272.
+// Rows from which row-major weights (tiled image, K a multiple of 4) take a
+// GEMM instead of the GEMV's launches of 1 and 2 rows, each of which reads and
+// converts the whole weight: the f16 matrix-core GEMM (qi_gemm_rm.hip, f16
+// scales) from kRmMinRows, and where the scales rule it out the f32 one
+// (rm_gemm_kernel) from kRmGemmMinRows. Calls run in chunks of
+// kRmGemmChunkRows rows; partial sums take at most kRmPartFloats. MI355X, us
+// per call at 2 rows, GEMV / f16 GEMM: Q8_0 4096 x 4096 14.8 / 13.8, Q4_K 4096
+// x 14336 28.0 / 22.9, Q6_K 4096 x 14336 30.2 / 25.2, Q4_0 4096 x 12288 20.8 /
+// 20.5, Q4_0 200 x 512 8.4 / 8.4; f32 GEMM (Q4_K 4096 x 14336) 36.4 at 2 rows,
+// 37.7 at 4, where the GEMV's two launches take 54.7.
+constexpr uint64_t kRmMinRows = 2;
 constexpr uint64_t kRmGemmMinRows = 3;
 constexpr uint64_t kRmGemmChunkRows = 4096;
 constexpr uint64_t kRmPartFloats = 8ull << 20;
@@ -221,13 +223,16 @@ constexpr uint64_t kSplitChunkRows = 4096;
 // within p->part_floats. Calls run in chunks; a shorter last chunk takes its
 // own part count (enqueue_linear asks again).
 void plan_parts(const Image& im, uint64_t m, LinearPlan* p) {
-  const bool bf3 = p->kind == LinearPlan::kBf3Gemm;
-  const uint64_t rows = bf3 ? kBf3ChunkRows : kSplitChunkRows, chunk = m < rows ? m : rows;
+  const uint64_t rows = p->kind == LinearPlan::kBf3Gemm    ? kBf3ChunkRows
+                        : p->kind == LinearPlan::kRmGemm   ? kRmGemmChunkRows
+                                                           : kSplitChunkRows;
+  const uint64_t chunk = m < rows ? m : rows;
   p->s_floats = 0;
   for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
     if (r == 0) continue;
-    const uint32_t parts = bf3 ? qi::gemm_bf3_plan(im, r, p->part_floats).parts
-                               : qi::gemm_split_splits(im, r, p->part_floats);
+    const uint32_t parts = p->kind == LinearPlan::kBf3Gemm  ? qi::gemm_bf3_plan(im, r, p->part_floats).parts
+                           : p->kind == LinearPlan::kRmGemm ? qi::gemm_rm_plan(im, r, p->part_floats).parts
+                                                            : qi::gemm_split_splits(im, r, p->part_floats);
     if (parts > 1) p->s_floats = std::max(p->s_floats, static_cast<uint64_t>(parts) * r * im.n);
   }
 }
@@ -266,6 +271,12 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     p->kind = LinearPlan::kF32Gemv;
     p->splits = qi::f32w_splits(im);
     if (p->splits > 1) p->s_floats = static_cast<uint64_t>(p->splits) * (m < 8 ? m : 8) * im.n;
+    return QI_HIP_OK;
+  }
+  if (mode != QI_HIP_MODE_EXACT && qi::gemm_rm_supported(im) && m >= kRmMinRows) {
+    p->kind = LinearPlan::kRmGemm;
+    p->part_floats = kRmPartFloats;
+    plan_parts(im, m, p);
     return QI_HIP_OK;
   }
   if (mode != QI_HIP_MODE_EXACT && qi::rm_gemm_supported(im) && m >= kRmGemmMinRows) {
@@ -368,6 +379,14 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
         const uint64_t rows = m - m0 < kRmGemmChunkRows ? m - m0 : kRmGemmChunkRows;
         const uint32_t parts = qi::rm_gemm_parts(im, rows, kRmPartFloats);
         QI_HIP_TRY(qi::launch_rm_gemm(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, parts, st),
+                   "launch row-major GEMM");
+      }
+      return QI_HIP_OK;
+    case LinearPlan::kRmGemm:
+      for (uint64_t m0 = 0; m0 < m; m0 += kRmGemmChunkRows) {
+        const uint64_t rows = m - m0 < kRmGemmChunkRows ? m - m0 : kRmGemmChunkRows;
+        QI_HIP_TRY(qi::launch_gemm_rm(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws,
+                                      qi::gemm_rm_plan(im, rows, p.part_floats), st),
                    "launch row-major GEMM");
       }
       return QI_HIP_OK;

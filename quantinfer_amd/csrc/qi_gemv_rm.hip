@@ -1,9 +1,10 @@
 // Row-major (blocks along N) GEMV and GEMM, F32 mode: y[m, n] = sum_k x[m, k]
 // w(k, n) for QuantInfer-layout weights (backends/cpu/src/backend.rs:62-140 ->
-// matmul.rs:14-90; element values matmul.rs:162-280). From 3 rows on a tiled
-// image with K a multiple of 4 the call is rm_gemm_kernel (its comment below):
-// the records dequantized into LDS for the f32 matrix cores. The GEMV takes 1
-// and 2 rows, two kernels by image:
+// matmul.rs:14-90; element values matmul.rs:162-280). On a tiled image with K
+// a multiple of 4 the GEMV takes one row, and calls of more rows the f16
+// matrix-core GEMM (qi_gemm_rm.hip) or, where the scales are outside its range
+// (f32 block scales), from 3 rows rm_gemm_kernel below: the records dequantized
+// into LDS for the f32 matrix cores. Two GEMV kernels by image:
 //
 // Tiled image (N a multiple of 256; gemv_rmt_kernel): record (t, u) holds
 // rows k = 16t + c (c = 0..15) of outputs n = 256u + [0, 256), in the
@@ -178,16 +179,18 @@ __global__ __launch_bounds__(256) void gemv_rm_kernel(View v, const float* __res
   }
 }
 
-// y = sum of the K-split partials in split order; a sum that is not finite
+// y = sum of the K-split partials in a fixed order; a sum that is not finite
 // is recomputed in the reference's order
-template <int QT, bool WIDE>
+// (PAIRS: each eight in pairs, for the GEMM's up to 32 parts: the sums of 28,
+// Q6_K 14336 x 4096, added one by one left 1.7e-7 of the result, in pairs 1.4e-7)
+template <int QT, bool WIDE, bool PAIRS = false>
 __global__ __launch_bounds__(256) void rm_sum_kernel(const float* __restrict__ part, uint32_t splits,
                                                      uint64_t count, float* __restrict__ y, View v,
                                                      const float* __restrict__ x) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= count) return;
   // loads issued 8 at a time with no condition (past the last split the last
-  // one is read again and not added), ahead of the in-order adds
+  // one is read again and not added), ahead of the adds
   float s = 0.0f;
   for (uint32_t p0 = 0; p0 < splits; p0 += 8) {
     float t[8];
@@ -196,8 +199,14 @@ __global__ __launch_bounds__(256) void rm_sum_kernel(const float* __restrict__ p
       const uint32_t pj = p0 + j < splits ? p0 + j : splits - 1;
       t[j] = part[static_cast<uint64_t>(pj) * count + i];
     }
+    if constexpr (PAIRS) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s = p0 + j == 0 ? t[j] : p0 + j < splits ? s + t[j] : s;
+      for (int j = 0; j < 8; ++j) t[j] = p0 + j < splits ? t[j] : 0.0f;
+      s += ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s = p0 + j == 0 ? t[j] : p0 + j < splits ? s + t[j] : s;
+    }
   }
   if (!__builtin_isfinite(s)) s = exact_row_major_col<QT, WIDE>(v, x + (i / v.n) * v.k, i % v.n);
   y[i] = s;
@@ -630,6 +639,24 @@ hipError_t launch_rm_gemm_q(const View& v, const float* x, uint32_t m, float* y,
 }
 
 }  // namespace
+
+hipError_t launch_rm_sum(const Image& im, const View& v, const float* part, uint32_t splits, uint64_t count,
+                         float* y, const float* x, hipStream_t st) {
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0, st, part, splits, count,
+                       y, v, x);
+    return hipGetLastError();
+  };
+  const bool w = im.wide != 0;
+  switch (im.qtype) {
+    case kQ8_0: return w ? hipErrorInvalidValue : go(rm_sum_kernel<kQ8_0, false, true>);
+    case kQ4_0: return w ? hipErrorInvalidValue : go(rm_sum_kernel<kQ4_0, false, true>);
+    case kQ4_K: return w ? hipErrorInvalidValue : go(rm_sum_kernel<kQ4_K, false, true>);
+    case kQ5_K: return w ? hipErrorInvalidValue : go(rm_sum_kernel<kQ5_K, false, true>);
+    case kQ6_K: return w ? hipErrorInvalidValue : go(rm_sum_kernel<kQ6_K, false, true>);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 // 16-row tiles up to 16 rows, 32 above: 64-row tiles (one wavefront per
 // SIMD) ran 2-5% slower from 64 rows on (MI355X, Q4_K 4096 x 14336 M=512

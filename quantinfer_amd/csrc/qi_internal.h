@@ -113,8 +113,25 @@ uint32_t rm_gemm_parts(const Image& im, uint64_t m, uint64_t max_part_floats);
 hipError_t launch_rm_gemm(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
                           uint32_t parts, hipStream_t st);
 
-// y = the sum of `splits` partial results of `count` = m * n values in split
-// order; a non-finite sum is recomputed in the reference's order.
+// Row-major GEMM with f32 accuracy on the f16 matrix cores (qi_gemm_rm.hip):
+// tiled row-major images with f16 scales (Q8_0 / Q4_0: within f16_gemm's
+// range), K a multiple of 4. K is split into plan.parts (the partial sums in
+// `part`, parts * m * n floats, when parts > 1); non-finite outputs are
+// recomputed in the reference's order.
+struct RmPlan {
+  uint32_t tm = 0;  // a workgroup's rows: 16 tm
+  uint32_t parts = 1;
+};
+bool gemm_rm_supported(const Image& im);
+RmPlan gemm_rm_plan(const Image& im, uint64_t m, uint64_t max_part_floats);
+hipError_t launch_gemm_rm(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
+                          const RmPlan& plan, hipStream_t st);
+
+// y = the sum of `splits` partial results of `count` = m * n values in a fixed
+// order (launch_rm_sum: images with f16 scales); a non-finite sum is recomputed
+// in the reference's order.
+hipError_t launch_rm_sum(const Image& im, const View& v, const float* part, uint32_t splits, uint64_t count,
+                         float* y, const float* x, hipStream_t st);
 hipError_t launch_f32w_sum(const View& v, const float* part, uint32_t splits, uint64_t count, float* y,
                            const float* x, hipStream_t st);
 

@@ -203,6 +203,49 @@ def test_row_major_slice_weights_are_the_dequantized_ones(ctx, qtype):
 
 
 @pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+def test_row_major_gemm_tiles(ctx, qtype):
+    """The row-major GEMM at the edges of its tiles: less than one 32-row stage
+    of k, partial last stages and 64-row chunks, row counts at and past every
+    tile height, K parts and none; within the F32 bars and deterministic."""
+    for k, n in ((4, 256), (36, 512), (100, 256), (1028, 768), (2304, 2048)):
+        blocks = po.make_weights(qtype, n, k, seed=2360 + qtype + k, outliers=qtype >= qa.Q4_K)
+        w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+        for m in (2, 16, 17, 33, 49, 64, 65, 130):
+            x = po.fill_normal(3360 + m + k, m * k).reshape(m, k)
+            y = w.linear(x, qa.MODE_F32)
+            _assert_f32_row_major(y, x, blocks, qtype, n, (k, n, m))
+            assert w.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+        w.free()
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+def test_row_major_gemm_scaled_rows(ctx, qtype):
+    """Activation rows of very different magnitudes (1e-6 to 1e4) in one call
+    and rows with one activation 1e4 times the others: each (row, 64 k) takes
+    its own power of two, so every row keeps the relative F32 bars (1) and
+    (2). Q8_0 / Q4_0 scales below f16's normal range take the f32 GEMM."""
+    k, n, m = 1088, 512, 40
+    blocks = po.make_weights(qtype, n, k, seed=2380 + qtype, outliers=qtype >= qa.Q4_K)
+    x = po.fill_normal(3380, m * k).reshape(m, k) * (10.0 ** np.linspace(-6, 4, m)).astype(np.float32)[:, None]
+    x[::3, 77] *= np.float32(1e4)
+    for small in (False, True):
+        if small:
+            blocks["scale"] = (blocks["scale"] * np.float32(2.0 ** -12)).astype(np.float16).astype(np.float32)
+            if "min_scale" in blocks.dtype.names:
+                blocks["min_scale"] = (blocks["min_scale"] * np.float32(2.0 ** -12)).astype(np.float16).astype(np.float32)
+        w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+        assert w.info().f16_scales == 1
+        d = po.dequantize(qtype, blocks).reshape(k, n)
+        y = w.linear(x, qa.MODE_F32)
+        exact = x.astype(np.float64) @ d.astype(np.float64)
+        cpu = po.matmul_row_major(qtype, x, blocks, n)
+        comp = guarded_rel_err(y, exact, x, d.T)
+        norm = max(normwise_rel_err(y[i], cpu[i]) for i in range(m))
+        assert comp <= F32_TOL and norm <= F32_TOL, (small, comp, norm)
+        w.free()
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
 def test_row_major_f32_block_scales(ctx, qtype):
     """Row-major tiled images with f32 block scales (random codes, scales not
     f16-exact): F32 mode within the bars with one split (K = 48) and with a
