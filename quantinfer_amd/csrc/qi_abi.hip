@@ -178,17 +178,14 @@ struct LinearPlan {
 };
 
 // Rows from which row-major weights (tiled image, K a multiple of 4) take a
-// GEMM instead of the GEMV's launches of 1 and 2 rows, each of which reads and
-// converts the whole weight: the f16 matrix-core GEMM (qi_gemm_rm.hip, f16
-// scales) from kRmMinRows, and where the scales rule it out the f32 one
-// (rm_gemm_kernel) from kRmGemmMinRows. Calls run in chunks of
-// kRmGemmChunkRows rows; partial sums take at most kRmPartFloats. MI355X, us
-// per call at 2 rows, GEMV / f16 GEMM: Q8_0 4096 x 4096 14.8 / 13.8, Q4_K 4096
-// x 14336 28.0 / 22.9, Q6_K 4096 x 14336 30.2 / 25.2, Q4_0 4096 x 12288 20.8 /
-// 20.5, Q4_0 200 x 512 8.4 / 8.4; f32 GEMM (Q4_K 4096 x 14336) 36.4 at 2 rows,
-// 37.7 at 4, where the GEMV's two launches take 54.7.
-constexpr uint64_t kRmMinRows = 2;
-constexpr uint64_t kRmGemmMinRows = 3;
+// GEMM instead of the GEMV's launches of up to 4 rows: the f16 matrix-core GEMM
+// (qi_gemm_rm.hip, f16 scales), or where the scales rule it out the f32 one
+// (rm_gemm_kernel). Calls run in chunks of kRmGemmChunkRows rows; partial sums
+// take at most kRmPartFloats. MI355X, us per call, GEMV at 4 rows / f16 GEMM at
+// 5: Q8_0 4096 x 4096 10.7 / 13.2, Q4_K 4096 x 14336 17.5 / 25.9, Q6_K 14336 x
+// 4096 25.7 / 27.5, Q4_0 4096 x 12288 15.7 / 21.0, Q5_K 1024 x 1024 10.0 / 9.1;
+// the f32 GEMM takes 35.1 at 4 rows of Q4_K 4096 x 14336.
+constexpr uint64_t kRmGemmMinRows = 5;
 constexpr uint64_t kRmGemmChunkRows = 4096;
 constexpr uint64_t kRmPartFloats = 8ull << 20;
 
@@ -273,7 +270,7 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     if (p->splits > 1) p->s_floats = static_cast<uint64_t>(p->splits) * (m < 8 ? m : 8) * im.n;
     return QI_HIP_OK;
   }
-  if (mode != QI_HIP_MODE_EXACT && qi::gemm_rm_supported(im) && m >= kRmMinRows) {
+  if (mode != QI_HIP_MODE_EXACT && qi::gemm_rm_supported(im) && m >= kRmGemmMinRows) {
     p->kind = LinearPlan::kRmGemm;
     p->part_floats = kRmPartFloats;
     plan_parts(im, m, p);

@@ -1,7 +1,7 @@
 // Row-major (blocks along N) GEMM on the f16 matrix cores with f32 accuracy:
 // y[m, n] = sum_k x[m, k] w(k, n) for QuantInfer-layout weights
 // (backends/cpu/src/backend.rs:62-140 -> matmul.rs:14-90; element values
-// matmul.rs:162-280), 2 rows and more, tiled images with f16 scales.
+// matmul.rs:162-280), 5 rows and more, tiled images with f16 scales.
 //
 // Arithmetic (the split halves of qi_half.h, with the scales that change along
 // k on the activations' side). A weight is d s (q - z) - b', with d the scale
@@ -39,7 +39,7 @@
 // 38 matrix instructions of 16 cycles), which slow down from 5 to 8-11 cycles
 // each while the other wavefront of a SIMD runs matrix instructions. MI355X, us
 // per call, the f32 matrix-core kernel (wide scales still take it) -> this one:
-// Q8_0 4096 x 4096 2 rows (the GEMV) 14.8 -> 13.8, 16 16.8 -> 14.4, 64 32.9 ->
+// Q8_0 4096 x 4096 5 rows 15.7 -> 13.2, 16 16.8 -> 14.4, 64 32.9 ->
 // 26.2, 130 65.2 -> 40.4, 512 170 -> 94; Q4_K 4096 x 14336 16 rows 36.8 -> 28.0,
 // 130 235 -> 99, 512 655 -> 299; Q4_0 4096 x 12288 2048 rows 1911 -> 765.
 #include "qi_device.h"

@@ -1,25 +1,37 @@
 // Row-major (blocks along N) GEMV and GEMM, F32 mode: y[m, n] = sum_k x[m, k]
 // w(k, n) for QuantInfer-layout weights (backends/cpu/src/backend.rs:62-140 ->
 // matmul.rs:14-90; element values matmul.rs:162-280). On a tiled image with K
-// a multiple of 4 the GEMV takes one row, and calls of more rows the f16
-// matrix-core GEMM (qi_gemm_rm.hip) or, where the scales are outside its range
-// (f32 block scales), from 3 rows rm_gemm_kernel below: the records dequantized
-// into LDS for the f32 matrix cores. Two GEMV kernels by image:
+// a multiple of 4 calls of 5 rows and more take the f16 matrix-core GEMM
+// (qi_gemm_rm.hip) or, where the scales are outside its range (f32 block
+// scales), rm_gemm_kernel below: the records dequantized into LDS for the f32
+// matrix cores. Two GEMV kernels by image:
 //
-// Tiled image (N a multiple of 256; gemv_rmt_kernel): record (t, u) holds
-// rows k = 16t + c (c = 0..15) of outputs n = 256u + [0, 256), in the
-// arrangement of the output-rows records. Lane 16g + c of a wavefront loads row
-// c's lane group g with the GEMV's record loader (Unit<QT>, non-temporal): the
-// codes of 64 outputs at one k and the scales of their windows. The lane keeps
-// one f32 accumulator per output and activation row and adds x[k] w per code
-// (rmt_consume: the codes centred as the one-row output-rows GEMV takes them,
-// the weight formed in one multiply-add where an offset is left).
-// A workgroup of four wavefronts takes one unit and one K split, each
-// wavefront every fourth tile of the split: at most rmt_max_slots records,
-// all loaded before the first is consumed.
-// The 16 rows of a lane group are summed by two DPP steps (lanes c, c + 4,
-// c + 8, c + 12) and through LDS for the last four and the four wavefronts, in
-// a fixed order.
+// Tiled image (N a multiple of 256; gemv_rmd_kernel, 1 to 4 rows): record
+// (t, u) holds rows k = 16t + c (c = 0..15) of outputs n = 256u + [0, 256), in
+// the arrangement of the output-rows records. Along N the scales change with
+// k, the index that is summed, so they go on the activations' side and the
+// codes to the int8 matrix cores: per 64 k and sub-block (outputs that share a
+// scale), F = rint(x a 2^s), 30 bits of the largest |x a|, is cut into four
+// signed 8-bit digits and v_mfma_i32_16x16x64_i8 multiplies the digits of up
+// to four rows (16 rows of A) by the codes of 16 outputs, exactly. Codes are
+// centred, Q4_K/Q5_K on a zero point per (k, window), whose small offset
+// b - a z is summed in f32 beside them. Both operands need 64 k of one output in
+// a lane, the records hold 64 outputs of one k: a wavefront writes its codes
+// and digits to its own LDS area in row order and reads them back with
+// transposing reads (ds_read_b64_tr_b8); row strides of 144 bytes keep both
+// sides free of bank conflicts. A workgroup of four wavefronts takes one unit
+// and one K split, each wavefront every fourth chunk of 64 k, at most two, all
+// loaded before the first is used; the wavefronts' sums are added through LDS,
+// the splits by rm_sum_kernel.
+// 1351 vector instructions per wavefront of 8 records at one Q4_K row, where a
+// conversion and two f32 multiply-adds per code took 2351. MI355X, us per call
+// (one launch of 1 row, 2-row launches or from 3 rows the f32 GEMM before ->
+// now): Q4_K 4096 x 14336 1 row 15.7 -> 14.0, 2 28.4 -> 15.2, 4 35.1 -> 17.5;
+// Q5_K 1 row 17.3 -> 16.1; Q6_K 14336 x 4096 1 row 21.0 -> 18.9, 4 37.0 -> 25.7;
+// Q4_0 4096 x 12288 2 rows 20.8 -> 13.4; Q8_0 4096 x 4096 4 rows 15.4 -> 10.7.
+// Error against 64-bit sums 0.9e-7 at K = 4096 (1.2e-7 to 1.4e-7 before). Of the
+// 14.0 us the kernel takes 10 and the split sum's launch and round trip the
+// rest.
 //
 // Planar image (gemv_rm_kernel): flat block index k * (N / bs) + nb, so at
 // one k the code bytes of consecutive output blocks are contiguous. A lane
@@ -37,6 +49,8 @@
 #include "qi_device.h"
 #include "qi_internal.h"
 #include "qi_unit.h"
+
+#include <type_traits>
 
 namespace qi {
 
@@ -214,185 +228,255 @@ __global__ __launch_bounds__(256) void rm_sum_kernel(const float* __restrict__ p
 
 // ------------------------------------------------------------ tiled image
 
-constexpr int kRmtRows = 2;     // activation rows per launch
-constexpr int kRmtStride = 17;  // float4s per summed lane in LDS: 64 outputs and one of padding
+constexpr int kRmtRows = 4;  // activation rows per launch
 
-// Records per wavefront, all loaded before the first is consumed (a record
-// in registers with its activation: Q4_0 11, Q4_K 14, Q8_0 and Q6_K 19, Q5_K
-// 22 VGPRs). Q4_0/Q4_K take 8 at two wavefronts per SIMD; the others 4 at
-// three, as 6 leaves them at two: Q5_K 4096 x 14336 M=1 24.4 us with 6 slots,
-// 19.0 with 4; Q6_K 23.6 / 19.1; Q4_K with 4 slots 16.6 against 15.9 (MI355X).
-constexpr uint32_t rmt_max_slots(int32_t qtype, uint32_t rows) {
-  return rows > 1 ? 4u : (qtype == kQ4_0 || qtype == kQ4_K) ? 8u : 4u;
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kRmdChunk = 64;          // weight rows of a chunk: one matrix-instruction step
+constexpr uint32_t kRmdWs = 128 + 16;       // LDS row stride of a chunk's codes (bytes)
+constexpr uint32_t kRmdCodes = kRmdChunk * kRmdWs;
+
+// Sub-blocks (one scale each) of a lane group's 32 outputs in a phase, and
+// LDS bytes of one wavefront: codes, digits [sub-block][k][16] and factors.
+template <int QT>
+constexpr uint32_t rmd_subs() {
+  return QT == kQ6_K ? 2 : 1;
+}
+template <int QT>
+struct RmdLds {
+  static constexpr uint32_t kDig = kRmdChunk * 16 + 8;  // digits of one sub-block, padded against conflicts
+  static constexpr uint32_t kSubs = 4 * rmd_subs<QT>();
+  static constexpr uint32_t kFac = kRmdCodes + kSubs * kDig;
+  static constexpr uint32_t kWave = kFac + kSubs * 4 * 8;
+  static_assert(kWave % 16 == 0, "aligned wavefront areas");
+};
+
+__device__ __forceinline__ uint32_t rmd_max(uint32_t v) {
+  auto step = [&](auto ctrl) {
+    const uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), decltype(ctrl)::value, 0xF, 0xF, false));
+    v = o > v ? o : v;
+  };
+  step(std::integral_constant<int, 0x121>{});
+  step(std::integral_constant<int, 0x122>{});
+  step(std::integral_constant<int, kDppRor4>{});
+  step(std::integral_constant<int, kDppRor8>{});
+  return v;
 }
 
-// Record of tile t into r, with the activations of its row k = 16t + c,
-// read at min(k, K - 1) (rows past K are zero in the record and their
-// activation is zeroed at use). No condition on loaded values here, so that
-// nothing waits for the loads before the record is consumed.
-template <int QT, bool WIDE, int MT>
-__device__ __forceinline__ void rmt_fetch(const uint8_t* rec, uint32_t lane, uint32_t k, uint32_t K,
-                                          const float* __restrict__ x, typename Unit<QT>::Raw& r,
-                                          float (&xs)[MT]) {
-  const uint32_t kk = k < K ? k : K - 1;
-#pragma unroll
-  for (int i = 0; i < MT; ++i) xs[i] = x[static_cast<uint64_t>(i) * K + kk];
-  Unit<QT>::template load<WIDE, true>(rec, lane, r);
-}
-
-// One record's products, acc[i][8 st + e] += x_i w for step st's code e. The
-// codes arrive centred, s (q - z) in a signed byte (one sign-extending
-// conversion); a / s is exact. Q8_0, Q4_0 and Q6_K have no offset left (w =
-// (a / s) s (q - z)): the lane forms x a / s once per window and multiplies.
-// Q4_K/Q5_K keep b - a z: the lane forms each weight with one fused
-// multiply-add, w = (a / s) s (q - z) - (b - a z), as a sum of x a q and of
-// x b over K would cancel in f32 at small K.
-template <int QT, bool WIDE, int MT>
-__device__ __forceinline__ void rmt_consume(const typename Unit<QT>::Raw& r, uint32_t g, bool live,
-                                            const float (&xr)[MT], float (&acc)[MT][64]) {
-  using U = Unit<QT>;
-  constexpr int kW = U::kWindows, kS = U::kSteps;
-  constexpr bool kOff = window_centered<QT>();
-  constexpr float kInv = 1.0f / static_cast<float>(code_scale<QT>());
-  constexpr float kCentre = static_cast<float>(code_centre<QT>());
-  float a[kW], b[kW], xa[MT][kW], xs[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) xs[i] = live ? xr[i] : 0.0f;
-  U::template scales<WIDE>(g, r, a, b);
-#pragma unroll
-  for (int w = 0; w < kW; ++w) {
-    if constexpr (kOff) {
-      b[w] = a[w] * kCentre - b[w];  // -(b - a z)
-      a[w] *= kInv;
-    } else {
-      const float as = a[w] * kInv;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) xa[i][w] = xs[i] * as;
-    }
-  }
-#pragma unroll
-  for (int st = 0; st < 8; ++st) {
-    const uint64_t q = static_cast<uint64_t>(gemv_codes<QT>(r, g, st));
-    const uint32_t lo = static_cast<uint32_t>(q), hi = static_cast<uint32_t>(q >> 32);
-    const int w = st / kS;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t word = e < 4 ? lo : hi;
-      const float qf = static_cast<float>(static_cast<int8_t>(word >> (8 * (e & 3))));
-      if constexpr (kOff) {
-        const float wt = fmaf(a[w], qf, b[w]);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i][8 * st + e] = fmaf(xs[i], wt, acc[i][8 * st + e]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i][8 * st + e] = fmaf(xa[i][w], qf, acc[i][8 * st + e]);
-      }
-    }
+// The 8 codes of step st as signed bytes s (q - z): Q4_K / Q5_K with the
+// zero point of their sub-block (t = (128 - z) in every byte, s = 1), the
+// other formats on the middle of their range (code_scale, code_centre).
+template <int QT>
+__device__ __forceinline__ uint64_t rmd_codes(const typename Unit<QT>::Raw& r, uint32_t g, int st, uint32_t t) {
+  if constexpr (window_centered<QT>()) {
+    const uint64_t q = static_cast<uint64_t>(Unit<QT>::codes(r, g, st));
+    const uint32_t lo = (static_cast<uint32_t>(q) + t) ^ 0x80808080u;
+    const uint32_t hi = (static_cast<uint32_t>(q >> 32) + t) ^ 0x80808080u;
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+  } else {
+    return static_cast<uint64_t>(gemv_codes<QT>(r, g, st));
   }
 }
 
 template <int QT, bool WIDE, int MT, int R>
-__global__ __launch_bounds__(256) void gemv_rmt_kernel(View v, const float* __restrict__ x, uint32_t m,
-                                                       uint32_t ksplit, float* __restrict__ out) {
+__global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* __restrict__ x, uint32_t m,
+                                                          uint32_t ksplit, float* __restrict__ out) {
   using U = Unit<QT>;
-  // [wavefront][row][lane group g * 4 + c, c < 4][64 outputs]
-  __shared__ float4 red[4][MT][16][kRmtStride];
+  using L = RmdLds<QT>;
+  constexpr int SW = rmd_subs<QT>(), NT = 2 / SW;  // sub-blocks per lane group and phase, 16-output tiles of each
+  constexpr bool kOff = window_centered<QT>();
+  constexpr float kInv = kOff ? 1.0f : 1.0f / static_cast<float>(code_scale<QT>());
+  extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar branches
-  const uint32_t K = static_cast<uint32_t>(v.k), T = v.tiles;
-  const uint32_t tb = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y) * T) / ksplit);
-  const uint32_t te = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y + 1) * T) / ksplit);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t K = static_cast<uint32_t>(v.k), T = v.tiles, C = (T + 3) / 4;
+  const uint32_t cb = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y) * C) / ksplit);
+  const uint32_t ce = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y + 1) * C) / ksplit);
   const uint8_t* base = v.qs + static_cast<uint64_t>(blockIdx.x) * v.rec.bytes;
   const uint64_t tile_bytes = static_cast<uint64_t>(v.units) * v.rec.bytes;
+  uint8_t* const wl = lds + wave * L::kWave;
 
-  float acc[MT][64];
+  float acc[2][4][2];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < 64; ++j) acc[i][j] = 0.0f;
-  // this wavefront's records: tiles t0, t0 + 4, ... below te, n <= R of them
-  // (the host picks the split count so). All R loads are issued first, with
-  // no condition (slots past n load the last record again), so that each
-  // record waits only for its own loads.
-  const uint32_t t0 = tb + wave, n = t0 < te ? (te - t0 + 3) / 4 : 0;
+  for (int j = 0; j < 16; ++j) acc[j >> 3][(j >> 1) & 3][j & 1] = 0.0f;
+
+  // this wavefront's chunks: cb + wave, cb + wave + 4, ... (at most R), the
+  // records of all of them loaded before the first is used, with no condition
+  // (chunks and tiles past the end load the last one again; their activations
+  // are zero)
+  const uint32_t c0 = cb + wave, n = c0 < ce ? (ce - c0 + 3) / 4 : 0;
   if (n > 0) {
-    typename U::Raw r[R];
-    float xs[R][MT];
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const uint32_t t = t0 + 4 * (static_cast<uint32_t>(j) < n ? j : n - 1);
-      rmt_fetch<QT, WIDE, MT>(base + t * tile_bytes, lane, 16 * t + c, K, x, r[j], xs[j]);
-      // loads in record order, all before the first record's arithmetic
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // every slot is consumed (no branch, so no load sinks into one): a slot
-    // past n, or a row past K, adds zero
+    typename U::Raw r[R][4];
+    float xs[R][4][MT];
 #pragma unroll
     for (int j = 0; j < R; ++j)
-      rmt_consume<QT, WIDE, MT>(r[j], g, static_cast<uint32_t>(j) < n && 16 * (t0 + 4 * j) + c < K, xs[j], acc);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint32_t tile = min(4 * (c0 + 4 * (static_cast<uint32_t>(j) < n ? j : n - 1)) + t, T - 1);
+        const uint32_t k = min(16 * tile + c, K - 1);
+#pragma unroll
+        for (int row = 0; row < MT; ++row)
+          xs[j][t][row] = x[static_cast<uint64_t>(min(static_cast<uint32_t>(row), m - 1)) * K + k];
+        U::template load<WIDE, true>(base + tile * tile_bytes, lane, r[j][t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if (static_cast<uint32_t>(j) >= n) break;
+      const uint32_t k0 = kRmdChunk * (c0 + 4 * j) + c;  // record t: row k0 + 16 t
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // scales of the phase's sub-blocks, their zero points and offsets
+        float a[4][SW], b[4][SW];
+        uint32_t zt[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          float aa[U::kWindows], bb[U::kWindows];
+          U::template scales<WIDE>(g, r[j][t], aa, bb);
+#pragma unroll
+          for (int i = 0; i < SW; ++i) a[t][i] = aa[h * SW + i];
+          if constexpr (kOff) {
+            // q - z stays a signed byte for codes up to 31
+            const float z = fmaxf(window_zero_point(aa[h], bb[h]), -96.0f);
+            b[t][0] = fmaf(-z, aa[h], bb[h]);
+            zt[t] = static_cast<uint32_t>(128 - static_cast<int>(z)) * 0x01010101u;
+          } else {
+            zt[t] = 0;
+          }
+        }
+        // digits of x a, 30 bits of the largest |x a| of the chunk
+#pragma unroll
+        for (int row = 0; row < MT; ++row) {
+          float xv[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) xv[t] = k0 + 16 * t < K ? xs[j][t][row] : 0.0f;
+#pragma unroll
+          for (int i = 0; i < SW; ++i) {
+            float p[4];
+            uint32_t mx = 0;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              p[t] = xv[t] * a[t][i];
+              const uint32_t bits = __builtin_bit_cast(uint32_t, p[t]) & 0x7FFFFFFFu;
+              mx = bits > mx ? bits : mx;
+            }
+            mx = rmd_max(mx);
+            const bool finite = mx < 0x7F800000u;
+            const float top = __builtin_bit_cast(float, mx);
+            const int e = finite && mx != 0 ? __builtin_amdgcn_frexp_expf(top) : 0;
+            const int sh = min(30 - e, 126);
+            uint8_t* const dig = wl + kRmdCodes + (g * SW + i) * L::kDig + 4 * row;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const int F = finite ? static_cast<int>(rintf(ldexpf(p[t], sh))) : 0;
+              const uint32_t d = (static_cast<uint32_t>(F) + 0x00808080u) ^ 0x00808080u;
+              *reinterpret_cast<uint32_t*>(dig + (16 * t + c) * 16) = d;
+            }
+            float off = 0.0f;
+            if constexpr (kOff) {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) off = fmaf(xv[t], b[t][0], off);
+              off += dpp_move<0x121>(off);
+              off += dpp_move<0x122>(off);
+              off += dpp_move<kDppRor4>(off);
+              off += dpp_move<kDppRor8>(off);
+            }
+            // NaN: every output of the row comes out non-finite and is
+            // recomputed in the reference's order
+            if (c == 0)
+              *reinterpret_cast<float2*>(wl + L::kFac + ((g * SW + i) * 4 + row) * 8) =
+                  make_float2(finite ? ldexpf(kInv, -sh) : __builtin_nanf(""), off);
+          }
+        }
+        // codes [k][128 outputs of the phase]
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          uint64_t q[4];
+#pragma unroll
+          for (int st = 0; st < 4; ++st) q[st] = rmd_codes<QT>(r[j][t], g, 4 * h + st, zt[t]);
+          ulonglong2* dst = reinterpret_cast<ulonglong2*>(wl + (16 * t + c) * kRmdWs + 32 * g);
+          dst[0] = make_ulonglong2(q[0], q[1]);
+          dst[1] = make_ulonglong2(q[2], q[3]);
+        }
+        // the wavefront's own LDS accesses complete in order: no wait beyond
+        // the reads' own
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        // k slots of both operands: lane group g, 8 g + [0, 8) and 32 + 8 g + [0, 8)
+        typedef __attribute__((address_space(3))) i32x2* lds_t;
+        auto tr = [&](const uint8_t* p0, uint32_t stride) {
+          const i32x2 lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0));
+          const i32x2 hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0 + 32 * stride));
+          return i32x4{lo[0], lo[1], hi[0], hi[1]};
+        };
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+#pragma unroll
+          for (int i = 0; i < SW; ++i) {
+            const i32x4 av = tr(wl + kRmdCodes + (w * SW + i) * L::kDig + (8 * g + (c >> 1)) * 16 + 8 * (c & 1), 16);
+            const float2 f = *reinterpret_cast<const float2*>(wl + L::kFac + ((w * SW + i) * 4 + g) * 8);
+#pragma unroll
+            for (int q = 0; q < NT; ++q) {
+              const int tile = SW == 2 ? i : q;
+              const i32x4 bv = tr(wl + (8 * g + (c >> 1)) * kRmdWs + 32 * w + 16 * tile + 8 * (c & 1), kRmdWs);
+              // lane 16 g + c: the four digit sums of row g, output c of the tile
+              const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
+              const float comb = fmaf(static_cast<float>(d[2] + 256 * d[3]), 65536.0f, static_cast<float>(d[0] + 256 * d[1]));
+              acc[h][w][tile] += kOff ? fmaf(comb, f.x, -f.y) : comb * f.x;
+            }
+          }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
   }
 
-  // rows c, c + 4, c + 8, c + 12 of each lane group, then lanes c < 4 to LDS
+  // the four wavefronts' sums [wave][row][256], added in wave order
+  __syncthreads();
+  float* const red = reinterpret_cast<float*>(lds);
+  if (g < static_cast<uint32_t>(MT)) {
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
-      acc[i][j] += dpp_move<kDppRor8>(acc[i][j]);
-      acc[i][j] += dpp_move<kDppRor4>(acc[i][j]);
-    }
-  if (c < 4) {
+      for (int w = 0; w < 4; ++w)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      float4* dst = red[wave][i][4 * g + c];
-#pragma unroll
-      for (int q = 0; q < 16; ++q)
-        dst[q] = make_float4(acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]);
-    }
+        for (int q = 0; q < 2; ++q)
+          red[(wave * MT + g) * 256 + window_first<QT>(w, h) + 16 * q + c] = acc[h][w][q];
   }
   __syncthreads();
-  // wavefront i sums activation row i: lane 16g + h takes outputs 4h .. 4h + 3
-  // of lane group g (step h / 2: elements window_first(g, h / 8) + 8 (h / 2 % 4)
-  // + 4 (h % 2) + [0, 4))
-  if (wave >= static_cast<uint32_t>(MT) || wave >= m) return;
-  const uint32_t h = c, step = h / 2;
-  float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const uint64_t col = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
 #pragma unroll
-  for (int wv = 0; wv < 4; ++wv)
+  for (int row = 0; row < MT; ++row) {
+    if (static_cast<uint32_t>(row) >= m) break;
+    float y = 0.0f;
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const float4 p = red[wv][wave][4 * g + cc][h];
-      s.x += p.x; s.y += p.y; s.z += p.z; s.w += p.w;
-    }
-  const uint32_t e0 = window_first<QT>(g, step / 4) + 8 * (step % 4) + 4 * (h % 2);
-  const uint64_t n0 = static_cast<uint64_t>(blockIdx.x) * 256 + e0;
-  float* dst = out + (static_cast<uint64_t>(blockIdx.y) * m + wave) * v.n + n0;
-  const float val[4] = {s.x, s.y, s.z, s.w};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float y = val[e];
+    for (int wv = 0; wv < 4; ++wv) y += red[(wv * MT + row) * 256 + threadIdx.x];
     // a NaN or infinite activation: the reference's order decides NaN or
     // +-Inf (with a K split, rm_sum_kernel checks the sum instead)
     if (ksplit == 1 && !__builtin_isfinite(y))
-      y = exact_row_major_col<QT, WIDE>(v, x + static_cast<uint64_t>(wave) * K, n0 + e);
-    dst[e] = y;
+      y = exact_row_major_col<QT, WIDE>(v, x + static_cast<uint64_t>(row) * K, col);
+    out[(static_cast<uint64_t>(blockIdx.y) * m + row) * v.n + col] = y;
   }
 }
 
+// Chunks of a wavefront, all loaded before the first is used.
+constexpr uint32_t kRmdChunks = 2;
+
 template <int QT, bool WIDE, int MT>
 hipError_t launch_rmt_rows(const View& v, const float* x, uint32_t m, float* out, uint32_t splits, hipStream_t st) {
-  // records per wavefront: ceil(ceil(T / splits) / 4), served by the smallest slot count that holds them
-  const uint32_t per = static_cast<uint32_t>(((v.tiles + splits - 1) / splits + 3) / 4);
-  const dim3 grid(v.units, splits);
+  // chunks per wavefront: ceil(ceil(C / splits) / 4)
+  const uint32_t chunks = (v.tiles + 3) / 4, per = ((chunks + splits - 1) / splits + 3) / 4;
+  constexpr uint32_t bytes = 4 * RmdLds<QT>::kWave;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, v, x, m, splits, out);
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3(v.units, splits), dim3(256), bytes, st, v, x, m, splits, out);
     return hipGetLastError();
   };
-  constexpr int kMax = static_cast<int>(rmt_max_slots(QT, MT));
-  if (per <= 2) return go(gemv_rmt_kernel<QT, WIDE, MT, 2>);
-  if (per <= 4) return go(gemv_rmt_kernel<QT, WIDE, MT, 4>);
-  if constexpr (kMax > 4) {
-    if (per <= kMax) return go(gemv_rmt_kernel<QT, WIDE, MT, kMax>);
-  }
+  if (per <= 1) return go(gemv_rmd_kernel<QT, WIDE, MT, 1>);
+  if (per <= kRmdChunks) return go(gemv_rmd_kernel<QT, WIDE, MT, kRmdChunks>);
   return hipErrorInvalidValue;
 }
 
@@ -400,9 +484,10 @@ template <int QT, bool WIDE>
 hipError_t launch_rmt_q(const View& v, const float* x, uint32_t m, float* y, float* part, uint32_t splits,
                         hipStream_t st) {
   float* out = splits > 1 ? part : y;
-  if (m != 1 && m != kRmtRows) return hipErrorInvalidValue;  // the kernel reads MT = m rows
-  hipError_t e = m == 1 ? launch_rmt_rows<QT, WIDE, 1>(v, x, m, out, splits, st)
-                        : launch_rmt_rows<QT, WIDE, kRmtRows>(v, x, m, out, splits, st);
+  if (m < 1 || m > kRmtRows) return hipErrorInvalidValue;
+  hipError_t e = m == 1   ? launch_rmt_rows<QT, WIDE, 1>(v, x, m, out, splits, st)
+                 : m == 2 ? launch_rmt_rows<QT, WIDE, 2>(v, x, m, out, splits, st)
+                          : launch_rmt_rows<QT, WIDE, 4>(v, x, m, out, splits, st);
   if (e != hipSuccess || splits == 1) return e;
   const uint64_t count = static_cast<uint64_t>(m) * v.n;
   hipLaunchKernelGGL((rm_sum_kernel<QT, WIDE>), dim3(static_cast<uint32_t>((count + 255) / 256)), dim3(256), 0,
@@ -719,18 +804,15 @@ bool gemv_rm_supported(const Image& im) {
 
 uint32_t gemv_rm_rows(const Image& im) { return im.tiled ? kRmtRows : 4; }
 
-uint32_t gemv_rm_splits(const Image& im, uint32_t m) {
+uint32_t gemv_rm_splits(const Image& im, uint32_t) {
   const uint32_t be = block_elems(im.qtype);
   if (im.tiled) {
     // About 512 workgroups (two wavefronts per SIMD on 256 CUs) give each
-    // wavefront ceil(T / (4 s)) records; that count is rounded up to a slot
-    // count of the kernel (2, 4 or the most), and s lowered to the fewest
-    // splits that keep it.
-    const uint64_t rmax = rmt_max_slots(im.qtype, m > 1 ? kRmtRows : 1);
-    const uint64_t s0 = (512 + im.units - 1) / im.units;
-    const uint64_t per = ((im.tiles + s0 - 1) / s0 + 3) / 4;
-    const uint64_t slots = per <= 2 ? 2 : per <= 4 ? 4 : rmax;
-    const uint64_t s = (im.tiles + 4 * slots - 1) / (4 * slots);
+    // wavefront one chunk of 64 k, or two at most; then the fewest splits that
+    // keep that.
+    const uint64_t chunks = (im.tiles + 3) / 4, s0 = (512 + im.units - 1) / im.units;
+    const uint64_t per = ((chunks + s0 - 1) / s0 + 3) / 4 <= 1 ? 1 : kRmdChunks;
+    const uint64_t s = (chunks + 4 * per - 1) / (4 * per);
     return static_cast<uint32_t>(s < 1 ? 1 : s);
   }
   // enough K splits for about 1024 workgroups, keeping at least 16 k per

@@ -203,6 +203,23 @@ def test_row_major_slice_weights_are_the_dequantized_ones(ctx, qtype):
 
 
 @pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+def test_row_major_gemv_rows(ctx, qtype):
+    """The row-major GEMV of 1 to 4 rows (and K not a multiple of 4, where it
+    takes every row count) around its 16-row tiles and 64-row chunks, one chunk
+    per wavefront and two, with and without K splits; within the F32 bars.
+    K = 1: one product per output."""
+    for k, n in ((1, 256), (15, 256), (63, 512), (65, 256), (258, 768), (1100, 512), (8260, 256)):
+        blocks = po.make_weights(qtype, n, k, seed=2390 + qtype + k, outliers=qtype >= qa.Q4_K)
+        w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+        for m in (1, 2, 3, 4, 7):
+            x = po.fill_normal(3390 + m + k, m * k).reshape(m, k)
+            y = w.linear(x, qa.MODE_F32)
+            _assert_f32_row_major(y, x, blocks, qtype, n, (k, n, m))
+            assert w.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+        w.free()
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
 def test_row_major_gemm_tiles(ctx, qtype):
     """The row-major GEMM at the edges of its tiles: less than one 32-row stage
     of k, partial last stages and 64-row chunks, row counts at and past every
