@@ -72,14 +72,17 @@ constexpr uint32_t kSCopies = (kSStage + 1023) / 1024;   // 1 KB copies per stag
 constexpr uint32_t kSCUs = 256;                          // compute units of an MI355X (gfx950)
 static_assert(kSStage % 16 == 0 && 2 * kSStage <= 160 * 1024, "two stages fit LDS");
 
-// One (64-row tile, unit) stage per workgroup (split_stage).
+// One (64-row tile, unit) stage over gridDim.y workgroups (split_stage: 8
+// passes of 8 rows each).
 template <bool ORDER6>
 __global__ __launch_bounds__(256) void split_prep_kernel(const float* __restrict__ x, uint32_t K, uint64_t M,
                                                          uint8_t* __restrict__ rec) {
   const uint32_t units = K / 256;
   const uint64_t mt = blockIdx.x / units;
   const uint32_t u = blockIdx.x % units;
-  split_stage<kSRows, ORDER6>(x, K, M, mt * kSRows, u, rec + (mt * units + u) * kSStage);
+  const uint32_t passes = kSRows / 8 / gridDim.y;
+  split_stage<kSRows, ORDER6>(x, K, M, mt * kSRows, u, rec + (mt * units + u) * kSStage, blockIdx.y * passes,
+                              (blockIdx.y + 1) * passes);
 }
 
 struct SplitArgs {
@@ -330,12 +333,17 @@ hipError_t launch_gemm_split(const Image& im, const View& v, const float* x, uin
   const uint64_t gt = split_group_tiles();
   const uint64_t groups = (im.tiles + gt - 1) / gt;
   if (mtiles * units > 0x7fffffffull || mtiles > 0xFFFFFFu || groups > 0xFFFFFFu) return hipErrorInvalidValue;
+  // A stage's eight passes wait for their loads one after another; with fewer
+  // stages than about eight workgroups per CU they are dealt to several
+  // workgroups (1, 2, 4 or 8 passes each). 96 stages (333 x 4096): kernel 10.2
+  // -> 4.9 us; 80 (300 x 4096) 8.3 -> 5.2; 240 (300 x 12288) 9.0 -> 7.7 (MI355X).
+  const uint64_t stages = mtiles * units;
+  const uint32_t per_stage = stages >= 2048 ? 1 : stages >= 1024 ? 2 : stages >= 512 ? 4 : 8;
+  const dim3 grid(static_cast<uint32_t>(stages), per_stage);
   if (im.qtype == kQ6_K)
-    hipLaunchKernelGGL(split_prep_kernel<true>, dim3(static_cast<uint32_t>(mtiles * units)), dim3(256), 0, st, x,
-                       static_cast<uint32_t>(im.k), m, rec);
+    hipLaunchKernelGGL(split_prep_kernel<true>, grid, dim3(256), 0, st, x, static_cast<uint32_t>(im.k), m, rec);
   else
-    hipLaunchKernelGGL(split_prep_kernel<false>, dim3(static_cast<uint32_t>(mtiles * units)), dim3(256), 0, st, x,
-                       static_cast<uint32_t>(im.k), m, rec);
+    hipLaunchKernelGGL(split_prep_kernel<false>, grid, dim3(256), 0, st, x, static_cast<uint32_t>(im.k), m, rec);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const SplitArgs a{v, x, y, m, rec, static_cast<uint32_t>(mtiles), static_cast<uint32_t>(groups), splits, part};
