@@ -902,6 +902,7 @@ struct qi_hip_kv_cache {
   int32_t* tok = nullptr;   // [cap + 1]
   uint32_t* len_dev = nullptr;
   uint64_t len = 0;         // host mirror of *len_dev
+  uint64_t pos = 0;         // position of the rows being enqueued (prompt forwards)
   // attention partials for row batches of `rb` rows
   float *pm = nullptr, *pl = nullptr, *po = nullptr;
   uint32_t* tickets = nullptr;  // [rb][kv head], zero between launches
@@ -1080,7 +1081,23 @@ qi_hip_status attention(qi_hip_qwen3* m, qi_hip_kv_cache* c, uint32_t layer, uin
   a.keys_w = c->keys + layer * lay;
   a.values_w = c->values + layer * lay;
   a.tickets = c->tickets;
-  if (!fused && hd == 128 && !m->attn_fma) {
+  // Prompt rows of head_dim 128: the matrix-core kernel walks the context's
+  // chunks one after another, 7 us each, in one workgroup per (16 rows, KV
+  // head); the FMA kernel gives every (chunk, KV head, 16 query rows) a
+  // workgroup of its own and merges them, about 14 us a launch and 0.02 us a
+  // workgroup. A few rows against a long context (a conversation's next turn)
+  // are faster on the second: 8 KV heads, 355 positions, 2 to 16 rows 37.8 ->
+  // 17.5 us, 32 44.2 -> 22.8, 48 45.3 -> 29.0; 300 rows 38 against 80 (MI355X).
+  const uint32_t live = static_cast<uint32_t>((c->pos + rows + kChunk - 1) / kChunk);
+  bool fma = m->attn_fma;
+  if (!fused && hd == 128 && !fma) {
+    const uint64_t blocks = static_cast<uint64_t>((rows + 15) / 16) * k.num_key_value_heads;
+    const uint64_t row_blocks = (rows * group + 15) / 16;
+    const uint64_t mfma_us = 7 * live * ((blocks + 255) / 256);
+    const uint64_t fma_us = 14 * ((rows + c->rb - 1) / c->rb) + live * k.num_key_value_heads * row_blocks / 50;
+    fma = fma_us < mfma_us;
+  }
+  if (!fused && hd == 128 && !fma) {
     // prompt rows on the matrix cores: every row in one launch
     a.row0 = 0;
     a.nrows = rows;
@@ -1110,7 +1127,7 @@ qi_hip_status attention(qi_hip_qwen3* m, qi_hip_kv_cache* c, uint32_t layer, uin
                          dim3(64 * kAttnWaves), one_, st, b);                                    \
     else                                                                                         \
       hipLaunchKernelGGL((attn_kernel<HD_, G_, false, RB_>),                                     \
-                         dim3(a.chunks, a.kv_heads, (nr + RB_ - 1) / RB_), dim3(64 * kAttnWaves), \
+                         dim3(live, a.kv_heads, (nr + RB_ - 1) / RB_), dim3(64 * kAttnWaves), \
                          blk_, st, b);                                                           \
   } else
     QI_ATTN(128, 1) QI_ATTN(128, 2) QI_ATTN(128, 4) QI_ATTN(128, 8)
@@ -1347,6 +1364,7 @@ qi_hip_status forward_locked(qi_hip_qwen3* m, qi_hip_kv_cache* c, const int32_t*
   for (uint64_t r0 = 0; r0 < count; r0 += kMaxRows) {
     const uint32_t rows = static_cast<uint32_t>(count - r0 < kMaxRows ? count - r0 : kMaxRows);
     const bool last = r0 + rows == count;
+    c->pos = c->len + r0;
     if ((s = enqueue_forward(m, c, rows, last)) != QI_HIP_OK) return s;
   }
   c->len += count;

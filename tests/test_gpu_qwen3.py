@@ -270,6 +270,35 @@ def test_head_dim_128_prefill_row_blocks(qa, ctx, kernel, monkeypatch):
     dev.free()
 
 
+@pytest.mark.parametrize("heads", [8, 2])
+def test_few_rows_against_a_context(qa, ctx, heads, monkeypatch):
+    """Prompt rows of head_dim 128 after a context take the kernel that deals
+    the context's chunks to workgroups when they are few, the matrix-core one
+    otherwise (a fresh prompt, many rows); the logits equal those with every
+    prompt on the first within f32 rounding (1e-5 of the largest: two orders of
+    the same f32 sums), at context lengths around the 64-position chunks."""
+    cfg = small_config(hidden_size=512, intermediate_size=512, num_attention_heads=heads,
+                       num_key_value_heads=2, head_dim=128, vocab_size=384, max_position_embeddings=512)
+    w = Qwen3Weights(cfg, seed=0xA77)
+    out = {}
+    for env in (None, "1"):
+        if env:
+            monkeypatch.setenv("QI_HIP_QWEN3_ATTN_FMA", env)
+        m = w.device_model(ctx)
+        monkeypatch.delenv("QI_HIP_QWEN3_ATTN_FMA", raising=False)
+        got = []
+        for context, rows in ((63, 2), (64, 7), (190, 16), (191, 17), (257, 40), (200, 130)):
+            cache = m.kv_cache(420)
+            tok = np.random.default_rng(context).integers(0, 384, context + rows).astype(np.int32)
+            m.forward(cache, tok[:context])
+            got.append(m.forward(cache, tok[context:])[0].copy())
+            cache.free()
+        out[env] = got
+        m.free()
+    for a, b in zip(out[None], out["1"]):
+        assert np.max(np.abs(a - b)) <= 1e-5 * np.max(np.abs(b))
+
+
 @pytest.mark.parametrize("group", [1, 2, 8])
 def test_head_dim_128_prompt_attention_groups(qa, ctx, group):
     """F32 mode, head_dim 128, 1/2/8 query heads per KV head: a 100-row
