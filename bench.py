@@ -428,7 +428,7 @@ def gemm_bench(qtype: int, m: int, k: int, n: int, steps: int, warmup: int, mode
     }
 
 
-MFMA_F32_PEAK_TFLOPS = 157.3
+BF3_PEAK_TFLOPS = MFMA_F16_PEAK_TFLOPS / 6
 
 
 def f32_head_bench(steps: int, warmup: int) -> dict:
@@ -436,8 +436,8 @@ def f32_head_bench(steps: int, warmup: int) -> dict:
     the unchanged runtime's LM head, [4096, 151936] f32 (a Q6_K head is
     dequantized at load, runtime/src/qwen3/loader.rs:47-61). One decode row
     (the streaming F32 GEMV, HBM-bound on 2.49 GB), the 512-row prompt's
-    logits (the f32 matrix-core GEMM, f32w_gemm_kernel, against the f32
-    matrix-core peak), and the
+    logits (the GEMM on three exact bf16 pieces per number, gemm_bf3_kernel,
+    against a sixth of the bf16 matrix peak: six products each), and the
     synchronous per-token call with host buffers as the runtime makes it."""
     import quantinfer_amd as qa
     from quantinfer_amd import hiprt
@@ -483,9 +483,9 @@ def f32_head_bench(steps: int, warmup: int) -> dict:
         "m1_ms": round(out[1], 4),
         "roofline": {"bound": "hbm", "achieved": round(gbps, 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": round(gbps / HBM_PEAK_GBPS, 4), "traffic": None},
-        "m512": {"ms": round(out[512], 3), "tflops": round(tflops, 2), "kernel": "f32w_gemm_kernel (v_mfma_f32_16x16x4f32)",
-                 "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": MFMA_F32_PEAK_TFLOPS,
-                              "unit": "TFLOP/s", "frac": round(tflops / MFMA_F32_PEAK_TFLOPS, 4)}},
+        "m512": {"ms": round(out[512], 3), "tflops": round(tflops, 2), "kernel": "gemm_bf3_kernel (v_mfma_f32_16x16x32_bf16)",
+                 "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": round(BF3_PEAK_TFLOPS, 1),
+                              "unit": "TFLOP/s", "frac": round(tflops / BF3_PEAK_TFLOPS, 4)}},
         "through_abi_m1_ms": round(abi_ms, 4),
         "note": "through_abi: qi_hip_linear with host x and y (H2D 16 KB, GEMV, D2H 608 KB), the "
                 "per-token cost of the head when the unchanged runtime calls KernelBackend::matmul",
@@ -592,7 +592,7 @@ GEMV_POINTS = ([(0, 1, 4096, 4096, (1,))] +
 # The same points on row-major weights (QuantInfer layout, blocks along N:
 # backends/cpu/src/matmul.rs:14-90), the tiled row-major image: Q4_K at the
 # FFN up shape, Q4_0 at 4096 x 12288, Q8_0 at 4096^2, at their configs' row
-# counts (one row on the row-major GEMV, from 3 rows the row-major GEMM).
+# counts (1 to 4 rows on the row-major GEMV, from 5 the row-major GEMM).
 RM_POINTS = [(2, 3, 4096, 14336, (1, 8)), (1, 2, 4096, 12288, (1, 4, 16)), (0, 1, 4096, 4096, (1,))]
 # the prefill GEMM, Q8_0 and Q4_K, M x (K, N)
 GEMM_POINTS = [(3, q, k, n, (128, 512, 2048)) for q in (1, 3)
