@@ -648,6 +648,34 @@ def test_host_path_copy_regimes(ctx, qtype, m, k, n, note):
     w.free()
 
 
+@pytest.mark.parametrize("qtype,layout,m,k,n", [
+    (qa.F32, qa.ROW_MAJOR, 1, 3, 4),          # 3 floats: no whole 16-byte piece
+    (qa.F32, qa.ROW_MAJOR, 343, 3, 8),        # a block of 1024 floats, then 5
+    (qa.Q8_0, qa.OUTPUT_ROWS, 64, 4096, 64),  # 1 MiB: the largest read by a kernel
+    (qa.Q8_0, qa.OUTPUT_ROWS, 65, 4096, 64),  # copied
+])
+def test_host_activations_read_by_a_kernel(ctx, qtype, layout, m, k, n):
+    """Activations up to 1 MiB reach the device through a kernel that reads
+    the pinned buffer, larger ones through a copy: both give the result of
+    the device-buffer entry point bit for bit, twice with other values."""
+    from quantinfer_amd import hiprt
+    print(f"host activations {m}x{k}x{n}", flush=True)
+    blocks = (po.fill_normal(31, k * n, 0.02).reshape(k, n) if qtype == qa.F32
+              else po.make_weights(qtype, k, n, seed=31))
+    w = ctx.weights(qtype, layout, k, n, blocks)
+    stream = hiprt.Stream()
+    for seed in (32, 33):
+        x = po.fill_normal(seed, m * k).reshape(m, k)
+        xd, yd = hiprt.DeviceBuffer.from_array(x), hiprt.DeviceBuffer(m * n * 4)
+        w.linear_device(xd.ptr, m, yd.ptr, qa.MODE_AUTO, stream.handle)
+        stream.synchronize()
+        assert w.linear(x, qa.MODE_AUTO).tobytes() == yd.to_array(np.float32, (m, n)).tobytes()
+        xd.free()
+        yd.free()
+    stream.destroy()
+    w.free()
+
+
 def test_gpu_error_paths(ctx):
     blocks = po.make_weights(qa.Q8_0, 64, 4, seed=1)
     w = ctx.weights(qa.Q8_0, qa.OUTPUT_ROWS, 64, 4, blocks)
