@@ -185,6 +185,8 @@ struct LinearPlan {
   uint64_t m_pad = 0;
   uint32_t splits = 1;  // GEMM K splits, or row-major GEMV K splits per row chunk
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
+  uint64_t tail_rows = 0;    // kGemm: last rows that run as a launch of their own with K parts (tail_splits)
+  uint32_t tail_splits = 1;
   uint64_t part_floats = 0;  // kBf3Gemm, kSplitGemm: the most that partial sums may take
 };
 
@@ -266,6 +268,12 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     p->h_floats = (p->m_pad * im.k + 1) / 2;
     p->splits = qi::gemm_splits(im, m);
     if (p->splits > 1) p->s_floats = p->splits * p->m_pad * im.n;
+    p->tail_rows = qi::gemm_tail_rows(im, m, &p->tail_splits);
+    if (p->tail_rows > 0) {
+      // partial sums beside the f16 activations within the no-allocation entry point's scratch
+      p->s_floats = p->tail_splits * qi::gemm_padded_rows(p->tail_rows) * im.n;
+      if ((p->h_floats + p->s_floats) * 4 + 512 > kScratchBytes) p->tail_rows = p->s_floats = 0;
+    }
     return QI_HIP_OK;
   }
   if (mode != QI_HIP_MODE_EXACT && qi::f32w_gemv_supported(im)) {
@@ -363,6 +371,16 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
       if (silu_act != nullptr && silu_done != nullptr && ga.splits == 1 && qi::gemm_silu_supported(im)) {
         ga.act = silu_act;
         *silu_done = true;
+      } else if (p.tail_rows > 0) {
+        // whole rounds of workgroups first, then the last rows with K parts
+        const uint64_t head = m - p.tail_rows;
+        ga.m = ga.m_pad = head;
+        QI_HIP_TRY(qi::launch_gemm(im, ga, st), "launch gemm");
+        ga.x += head * im.k;
+        ga.y += head * im.n;
+        ga.m = p.tail_rows;
+        ga.m_pad = qi::gemm_padded_rows(ga.m);
+        ga.splits = p.tail_splits;
       }
       if (ga.splits > 1) ga.part = sws;
       QI_HIP_TRY(qi::launch_gemm(im, ga, st), "launch gemm");
@@ -485,6 +503,7 @@ qi_hip_status run_linear(qi_hip_ctx* c, const qi_hip_weights* w, const float* x,
     p.part_floats = bf3 ? 0 : c->scap;
     plan_parts(w->im, m, &p);
   }
+  if (p.tail_rows > 0 && p.s_floats > c->scap && capturing(st)) p.tail_rows = p.s_floats = 0;
   if ((s = grow_ws(c, st, &c->hbuf, &c->hcap, p.h_floats, "alloc GEMM workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->sbuf, &c->scap, p.s_floats, "alloc split-K workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->dbuf, &c->dcap, p.d_floats, "alloc GEMV workspace")) != QI_HIP_OK) return s;

@@ -1074,6 +1074,35 @@ uint32_t gemm_splits(const Image& im, uint64_t m) {
   return static_cast<uint32_t>(s < 1 ? 1 : s);
 }
 
+uint64_t gemm_tail_rows(const Image& im, uint64_t m, uint32_t* splits) {
+  // A last round of few workgroups takes as long as a full one. Its rows go to
+  // a second launch with K parts that fill the CUs, where the model says so:
+  // units of the longest chain x the time of a unit, against the second
+  // launch's activation and sum kernels and its partial sums' trip through
+  // memory. MI355X, us per call, one launch -> two: Q4_K 4096 x 12288 700 rows
+  // (288 blocks) 141.6 -> 120.5, 768 137.2 -> 118.8, 896 136.7 -> 129.1, 1300
+  // 198.7 -> 170.5, 1408 203.1 -> 180.7; Q8_0 4096 x 4096 2050 rows 134.6 ->
+  // 108.9, 2600 134.3 -> 126.2; Q5_K 4096 x 24576 700 rows 223.3 -> 205.7; Q4_0
+  // 2048 x 6144 1400 rows 77.6 -> 73.5, 1024 x 12288 768 rows 49.5 either way
+  // (one launch stays).
+  constexpr double kUnitUs = 4.2, kLaunchUs = 12.0, kPartUsPerByte = 0.37e-6;
+  constexpr uint64_t kCUs = 256;
+  *splits = 1;
+  const uint64_t nblk = (im.tiles + 15) / 16, mblk = gemm_padded_rows(m) / kTileM, units = im.k / 256;
+  const uint64_t rounds = nblk * mblk / kCUs;
+  const uint64_t head = rounds * kCUs / nblk;  // row blocks of the whole rounds
+  if (gemm_splits(im, m) != 1 || head == 0 || head >= mblk) return 0;
+  const uint64_t rows = m - head * kTileM;
+  const uint32_t s = gemm_splits(im, rows);
+  if (s == 1) return 0;
+  const double one = static_cast<double>((nblk * mblk + kCUs - 1) / kCUs * units) * kUnitUs;
+  const double two = static_cast<double>((nblk * head + kCUs - 1) / kCUs * units + (units + s - 1) / s) * kUnitUs +
+                     kLaunchUs + static_cast<double>(s * (mblk - head) * kTileM * im.n * 4) * kPartUsPerByte;
+  if (two >= one) return 0;
+  *splits = s;
+  return rows;
+}
+
 hipError_t launch_gemm(const Image& im, const GemmArgs& a, hipStream_t st) {
   if (!im.tiled || a.xh == nullptr || a.m_pad != gemm_padded_rows(a.m)) return hipErrorInvalidValue;
   if (use_ws(im.qtype)) {

@@ -187,6 +187,10 @@ uint64_t gemm_padded_rows(uint64_t m);
 // K splits of a GEMM launch (1: no split): enough workgroups to fill the CUs
 // once when the row and column blocks alone do not.
 uint32_t gemm_splits(const Image& im, uint64_t m);
+// Rows at the end of a call (0: none) that take a launch of their own with
+// *splits K parts, so that the rows before them (a multiple of 128) fill whole
+// rounds of the CUs.
+uint64_t gemm_tail_rows(const Image& im, uint64_t m, uint32_t* splits);
 // The GEMM kernel this image runs on has the SiLU-pairs epilogue.
 bool gemm_silu_supported(const Image& im);
 hipError_t launch_gemm(const Image& im, const GemmArgs& a, hipStream_t st);

@@ -755,6 +755,26 @@ def test_lds_gemm_both_kernels(ctx, qtype, m, monkeypatch):
     assert y_lds.tobytes() == y_reg.tobytes()
 
 
+@pytest.mark.parametrize("qtype", [qa.Q8_0, qa.Q4_0, qa.Q4_K, qa.Q5_K], ids=lambda q: NAMES[q])
+@pytest.mark.parametrize("m", [1025, 1100, 1152])
+def test_mfma_gemm_last_round(ctx, qtype, m):
+    """Rows past a whole round of the 256 CUs (1024 rows of 8192 outputs) run
+    as a launch of their own with K parts: the call's rows are bit for bit
+    those of the two calls, and its last rows meet the MFMA bars."""
+    k, n, head = 2048, 8192, 1024
+    print(f"last round {NAMES[qtype]} m={m}", flush=True)
+    blocks = po.make_weights(qtype, k, n, seed=6400 + qtype, outliers=True)
+    x = po.fill_normal(6500 + m, m * k).reshape(m, k)
+    w = ctx.weights(qtype, qa.OUTPUT_ROWS, k, n, blocks)
+    y = w.linear(x, qa.MODE_MFMA)
+    assert y[:head].tobytes() == w.linear(x[:head], qa.MODE_MFMA).tobytes()
+    assert y[head:].tobytes() == w.linear(x[head:], qa.MODE_MFMA).tobytes()
+    rows = np.array([head - 1, head, m - 1])
+    comp, norm, cpu = _mfma_checks(y[rows], np.ascontiguousarray(x[rows]), blocks, qtype, n)
+    assert comp <= MFMA_TOL and norm <= MFMA_TOL and cpu <= MFMA_TOL, (comp, norm, cpu)
+    w.free()
+
+
 def test_mfma_gemm_wide_scales(ctx):
     """f32 (not f16-exact) block scales through the GEMM, which rounds them to
     f16 operands; the scales stay in f16's normal range (beyond it the GEMM
