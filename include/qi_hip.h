@@ -162,8 +162,8 @@ qi_hip_status qi_hip_linear_device(qi_hip_ctx *ctx, const qi_hip_weights *w, con
  * QI_HIP_INVALID_INPUT (the f16 GEMM takes 2*M*K bytes of f16 activations, M
  * rounded up to 128, plus split-K partials when fewer than 256 row x column
  * blocks, or for the rows past the last whole 256 where they fit; the
- * split-half GEMM about 4.1*M*K bytes, M rounded up to 64 and at most 4096 per launch, and the K-part sums
- * that fit beside them). Every call on one GPU
+ * split-half GEMM about 4.1*M*K bytes, M rounded up to 64 and at most 4096 per
+ * launch, and the K-part sums that fit beside them). Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (other streams, other
  * threads, other contexts on the same device) race, and the caller must order
  * them. Nothing in the array needs clearing between calls. */
