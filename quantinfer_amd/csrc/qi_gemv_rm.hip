@@ -11,9 +11,15 @@
 // the arrangement of the output-rows records. Along N the scales change with
 // k, the index that is summed, so they go on the activations' side and the
 // codes to the int8 matrix cores: per 64 k and sub-block (outputs that share a
-// scale), F = rint(x a 2^s), 30 bits of the largest |x a|, is cut into four
+// scale), F = rint(x a 2^s), 30 bits below the largest |x a|, is cut into four
 // signed 8-bit digits and v_mfma_i32_16x16x64_i8 multiplies the digits of up
-// to four rows (16 rows of A) by the codes of 16 outputs, exactly. Codes are
+// to four (row, level) slots (16 rows of A) by the codes of 16 outputs,
+// exactly. What F leaves of x a makes the next level, times 2^31, until nothing
+// is left: two levels ride one instruction at one or two rows, more (in
+// practice at 3 and 4 rows, or past activations 2^37 times the others) repeat
+// it. So an activation far above the others takes no bits from them. (With the
+// first level alone, outputs with zero codes at an activation 1e6 times the
+// others had errors of 1.3e-4; now as without it.) Codes are
 // centred, Q4_K/Q5_K on a zero point per (k, window), whose small offset
 // b - a z is summed in f32 beside them. Both operands need 64 k of one output in
 // a lane, the records hold 64 outputs of one k: a wavefront writes its codes
@@ -23,15 +29,13 @@
 // and one K split, each wavefront every fourth chunk of 64 k, at most two, all
 // loaded before the first is used; the wavefronts' sums are added through LDS,
 // the splits by rm_sum_kernel.
-// 1351 vector instructions per wavefront of 8 records at one Q4_K row, where a
-// conversion and two f32 multiply-adds per code took 2351. MI355X, us per call
-// (one launch of 1 row, 2-row launches or from 3 rows the f32 GEMM before ->
-// now): Q4_K 4096 x 14336 1 row 15.7 -> 14.0, 2 28.4 -> 15.2, 4 35.1 -> 17.5;
-// Q5_K 1 row 17.3 -> 16.1; Q6_K 14336 x 4096 1 row 21.0 -> 18.9, 4 37.0 -> 25.7;
-// Q4_0 4096 x 12288 2 rows 20.8 -> 13.4; Q8_0 4096 x 4096 4 rows 15.4 -> 10.7.
-// Error against 64-bit sums 0.9e-7 at K = 4096 (1.2e-7 to 1.4e-7 before). Of the
-// 14.0 us the kernel takes 10 and the split sum's launch and round trip the
-// rest.
+// MI355X, us per call (one launch of 1 row, 2-row launches or from 3 rows the
+// f32 GEMM, f32 multiply-adds per code, before -> now): Q4_K 4096 x 14336 1 row
+// 16.1 -> 14.6, 2 27.7 -> 16.0, 4 34.8 -> 21.2; Q5_K 1 row 17.4 -> 16.7; Q6_K
+// 14336 x 4096 1 row 21.0 -> 19.8, 4 35.6 -> 31.1; Q4_0 4096 x 12288 2 rows 20.5
+// -> 14.3; Q8_0 4096 x 4096 4 rows 15.9 -> 12.2. (One level, 30 bits: Q4_K 14.0,
+// 15.1, 17.5.) Error against 64-bit sums 1.0e-7 at K = 4096 (1.4e-7 before). Of
+// the 14.6 us the split sum's launch and round trip take 4.
 //
 // Planar image (gemv_rm_kernel): flat block index k * (N / bs) + nb, so at
 // one k the code bytes of consecutive output blocks are contiguous. A lane
@@ -236,6 +240,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kRmdChunk = 64;          // weight rows of a chunk: one matrix-instruction step
 constexpr uint32_t kRmdWs = 128 + 16;       // LDS row stride of a chunk's codes (bytes)
 constexpr uint32_t kRmdCodes = kRmdChunk * kRmdWs;
+constexpr int kRmdMaxShift = 144;           // 2^-144 / code_scale is an f32 number
 
 // Sub-blocks (one scale each) of a lane group's 32 outputs in a phase, and
 // LDS bytes of one wavefront: codes, digits [sub-block][k][16] and factors.
@@ -285,6 +290,9 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
   using U = Unit<QT>;
   using L = RmdLds<QT>;
   constexpr int SW = rmd_subs<QT>(), NT = 2 / SW;  // sub-blocks per lane group and phase, 16-output tiles of each
+  constexpr int LV = MT <= 2 ? 2 : 1, Slots = MT * LV;  // levels in one matrix instruction (4 slots of 4 digits)
+  constexpr int SI = MT == 4 ? 1 : SW;  // sub-blocks at a time
+  constexpr int X = MT == 4 ? 1 : R;  // chunks of x loaded ahead: 256 registers hold no more
   constexpr bool kOff = window_centered<QT>();
   constexpr float kInv = kOff ? 1.0f : 1.0f / static_cast<float>(code_scale<QT>());
   extern __shared__ __align__(16) uint8_t lds[];
@@ -308,22 +316,29 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
   const uint32_t c0 = cb + wave, n = c0 < ce ? (ce - c0 + 3) / 4 : 0;
   if (n > 0) {
     typename U::Raw r[R][4];
-    float xs[R][4][MT];
+    float xs[X][4][MT];
+    auto load_x = [&](uint32_t tile, float (&o)[MT]) {
+      const uint32_t k = min(16 * tile + c, K - 1);
+#pragma unroll
+      for (int row = 0; row < MT; ++row)
+        o[row] = x[static_cast<uint64_t>(min(static_cast<uint32_t>(row), m - 1)) * K + k];
+    };
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const uint32_t tile = min(4 * (c0 + 4 * (static_cast<uint32_t>(j) < n ? j : n - 1)) + t, T - 1);
-        const uint32_t k = min(16 * tile + c, K - 1);
-#pragma unroll
-        for (int row = 0; row < MT; ++row)
-          xs[j][t][row] = x[static_cast<uint64_t>(min(static_cast<uint32_t>(row), m - 1)) * K + k];
+        if (j < X) load_x(tile, xs[j][t]);
         U::template load<WIDE, true>(base + tile * tile_bytes, lane, r[j][t]);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       if (static_cast<uint32_t>(j) >= n) break;
+      if (j >= X) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) load_x(min(4 * (c0 + 4 * j) + t, T - 1), xs[0][t]);
+      }
       const uint32_t k0 = kRmdChunk * (c0 + 4 * j) + c;  // record t: row k0 + 16 t
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -345,50 +360,6 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
             zt[t] = 0;
           }
         }
-        // digits of x a, 30 bits of the largest |x a| of the chunk
-#pragma unroll
-        for (int row = 0; row < MT; ++row) {
-          float xv[4];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) xv[t] = k0 + 16 * t < K ? xs[j][t][row] : 0.0f;
-#pragma unroll
-          for (int i = 0; i < SW; ++i) {
-            float p[4];
-            uint32_t mx = 0;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              p[t] = xv[t] * a[t][i];
-              const uint32_t bits = __builtin_bit_cast(uint32_t, p[t]) & 0x7FFFFFFFu;
-              mx = bits > mx ? bits : mx;
-            }
-            mx = rmd_max(mx);
-            const bool finite = mx < 0x7F800000u;
-            const float top = __builtin_bit_cast(float, mx);
-            const int e = finite && mx != 0 ? __builtin_amdgcn_frexp_expf(top) : 0;
-            const int sh = min(30 - e, 126);
-            uint8_t* const dig = wl + kRmdCodes + (g * SW + i) * L::kDig + 4 * row;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const int F = finite ? static_cast<int>(rintf(ldexpf(p[t], sh))) : 0;
-              const uint32_t d = (static_cast<uint32_t>(F) + 0x00808080u) ^ 0x00808080u;
-              *reinterpret_cast<uint32_t*>(dig + (16 * t + c) * 16) = d;
-            }
-            float off = 0.0f;
-            if constexpr (kOff) {
-#pragma unroll
-              for (int t = 0; t < 4; ++t) off = fmaf(xv[t], b[t][0], off);
-              off += dpp_move<0x121>(off);
-              off += dpp_move<0x122>(off);
-              off += dpp_move<kDppRor4>(off);
-              off += dpp_move<kDppRor8>(off);
-            }
-            // NaN: every output of the row comes out non-finite and is
-            // recomputed in the reference's order
-            if (c == 0)
-              *reinterpret_cast<float2*>(wl + L::kFac + ((g * SW + i) * 4 + row) * 8) =
-                  make_float2(finite ? ldexpf(kInv, -sh) : __builtin_nanf(""), off);
-          }
-        }
         // codes [k][128 outputs of the phase]
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
@@ -399,50 +370,125 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
           dst[0] = make_ulonglong2(q[0], q[1]);
           dst[1] = make_ulonglong2(q[2], q[3]);
         }
-        // the wavefront's own LDS accesses complete in order: no wait beyond
-        // the reads' own
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
-        // k slots of both operands: lane group g, 8 g + [0, 8) and 32 + 8 g + [0, 8)
-        typedef __attribute__((address_space(3))) i32x2* lds_t;
-        auto tr = [&](const uint8_t* p0, uint32_t stride) {
-          const i32x2 lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0));
-          const i32x2 hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0 + 32 * stride));
-          return i32x4{lo[0], lo[1], hi[0], hi[1]};
-        };
 #pragma unroll
-        for (int w = 0; w < 4; ++w)
+        for (int i0 = 0; i0 < SW; i0 += SI) {
+          // x a as fixed point: digits of level l are those of rint(t) for t = x a
+          // 2^sh, |t| < 2^30 at the first level and the remainder times 2^31 at
+          // each next one, until nothing is left of any product
+          float tt[MT][SI][4], ff[MT][SI];  // t of record t; the level's factor, NaN for a non-finite chunk
+          int sh[MT][SI];
+          float off[MT];
 #pragma unroll
-          for (int i = 0; i < SW; ++i) {
-            const i32x4 av = tr(wl + kRmdCodes + (w * SW + i) * L::kDig + (8 * g + (c >> 1)) * 16 + 8 * (c & 1), 16);
-            const float2 f = *reinterpret_cast<const float2*>(wl + L::kFac + ((w * SW + i) * 4 + g) * 8);
+          for (int row = 0; row < MT; ++row) {
+            float xv[4];
 #pragma unroll
-            for (int q = 0; q < NT; ++q) {
-              const int tile = SW == 2 ? i : q;
-              const i32x4 bv = tr(wl + (8 * g + (c >> 1)) * kRmdWs + 32 * w + 16 * tile + 8 * (c & 1), kRmdWs);
-              // lane 16 g + c: the four digit sums of row g, output c of the tile
-              const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
-              const float comb = fmaf(static_cast<float>(d[2] + 256 * d[3]), 65536.0f, static_cast<float>(d[0] + 256 * d[1]));
-              acc[h][w][tile] += kOff ? fmaf(comb, f.x, -f.y) : comb * f.x;
+            for (int t = 0; t < 4; ++t) xv[t] = k0 + 16 * t < K ? xs[j % X][t][row] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < SI; ++i) {
+              float p[4];
+              uint32_t mx = 0;
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                p[t] = xv[t] * a[t][i0 + i];
+                const uint32_t bits = __builtin_bit_cast(uint32_t, p[t]) & 0x7FFFFFFFu;
+                mx = bits > mx ? bits : mx;
+              }
+              mx = rmd_max(mx);
+              const bool finite = mx < 0x7F800000u;
+              const int e = finite && mx != 0 ? __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, mx)) : 0;
+              sh[row][i] = min(30 - e, kRmdMaxShift);
+              // NaN: every output of the row comes out non-finite and is
+              // recomputed in the reference's order
+              ff[row][i] = finite ? kInv : __builtin_nanf("");
+#pragma unroll
+              for (int t = 0; t < 4; ++t) tt[row][i][t] = finite ? ldexpf(p[t], sh[row][i]) : 0.0f;
+            }
+            off[row] = 0.0f;
+            if constexpr (kOff) {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) off[row] = fmaf(xv[t], b[t][0], off[row]);
+              off[row] += dpp_move<0x121>(off[row]);
+              off[row] += dpp_move<0x122>(off[row]);
+              off[row] += dpp_move<kDppRor4>(off[row]);
+              off[row] += dpp_move<kDppRor8>(off[row]);
             }
           }
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
+          for (bool more = true; more;) {
+            bool left = false;
+#pragma unroll
+            for (int l = 0; l < LV; ++l)
+#pragma unroll
+              for (int row = 0; row < MT; ++row)
+#pragma unroll
+                for (int i = 0; i < SI; ++i) {
+                  const int slot = l * MT + row, step = min(31, kRmdMaxShift - sh[row][i]);
+                  uint8_t* const dig = wl + kRmdCodes + (g * SI + i) * L::kDig + 4 * slot;
+                  float f[4];
+#pragma unroll
+                  for (int t = 0; t < 4; ++t) {
+                    f[t] = rintf(tt[row][i][t]);
+                    const uint32_t d = (static_cast<uint32_t>(static_cast<int>(f[t])) + 0x00808080u) ^ 0x00808080u;
+                    *reinterpret_cast<uint32_t*>(dig + (16 * t + c) * 16) = d;
+                  }
+                  if (c == 0)
+                    *reinterpret_cast<float2*>(wl + L::kFac + ((g * SI + i) * 4 + slot) * 8) =
+                        make_float2(ldexpf(ff[row][i], -sh[row][i]), off[row]);
+                  if constexpr (kOff) off[row] = 0.0f;
+#pragma unroll
+                  for (int t = 0; t < 4; ++t) {
+                    tt[row][i][t] = ldexpf(tt[row][i][t] - f[t], step);
+                    if (l == LV - 1) left |= tt[row][i][t] != 0.0f && step > 0;
+                  }
+                  sh[row][i] += step;
+                }
+            more = __any(left);
+            // the wavefront's own LDS accesses complete in order: no wait beyond
+            // the reads' own
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            // k slots of both operands: lane group g, 8 g + [0, 8) and 32 + 8 g + [0, 8)
+            typedef __attribute__((address_space(3))) i32x2* lds_t;
+            auto tr = [&](const uint8_t* p0, uint32_t stride) {
+              const i32x2 lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0));
+              const i32x2 hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_t)(p0 + 32 * stride));
+              return i32x4{lo[0], lo[1], hi[0], hi[1]};
+            };
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+#pragma unroll
+              for (int i = 0; i < SI; ++i) {
+                const i32x4 av = tr(wl + kRmdCodes + (w * SI + i) * L::kDig + (8 * g + (c >> 1)) * 16 + 8 * (c & 1), 16);
+                const float2 f = *reinterpret_cast<const float2*>(wl + L::kFac + ((w * SI + i) * 4 + g) * 8);
+#pragma unroll
+                for (int q = 0; q < NT; ++q) {
+                  const int tile = SW == 2 ? i0 + i : q;
+                  const i32x4 bv = tr(wl + (8 * g + (c >> 1)) * kRmdWs + 32 * w + 16 * tile + 8 * (c & 1), kRmdWs);
+                  // lane 16 g + c: the four digit sums of row g, output c of the tile
+                  const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
+                  const float comb = fmaf(static_cast<float>(d[2] + 256 * d[3]), 65536.0f, static_cast<float>(d[0] + 256 * d[1]));
+                  acc[h][w][tile] += kOff ? fmaf(comb, f.x, -f.y) : comb * f.x;
+                }
+              }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+          }
+        }
       }
     }
   }
 
-  // the four wavefronts' sums [wave][row][256], added in wave order
+  // the four wavefronts' sums [wave][level, row][256], the last level first, in
+  // wave order
   __syncthreads();
   float* const red = reinterpret_cast<float*>(lds);
-  if (g < static_cast<uint32_t>(MT)) {
+  if (g < static_cast<uint32_t>(Slots)) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int w = 0; w < 4; ++w)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
-          red[(wave * MT + g) * 256 + window_first<QT>(w, h) + 16 * q + c] = acc[h][w][q];
+          red[(wave * Slots + g) * 256 + window_first<QT>(w, h) + 16 * q + c] = acc[h][w][q];
   }
   __syncthreads();
   const uint64_t col = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -451,7 +497,9 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
     if (static_cast<uint32_t>(row) >= m) break;
     float y = 0.0f;
 #pragma unroll
-    for (int wv = 0; wv < 4; ++wv) y += red[(wv * MT + row) * 256 + threadIdx.x];
+    for (int l = LV - 1; l >= 0; --l)
+#pragma unroll
+      for (int wv = 0; wv < 4; ++wv) y += red[(wv * Slots + l * MT + row) * 256 + threadIdx.x];
     // a NaN or infinite activation: the reference's order decides NaN or
     // +-Inf (with a K split, rm_sum_kernel checks the sum instead)
     if (ksplit == 1 && !__builtin_isfinite(y))

@@ -219,6 +219,52 @@ def test_row_major_gemv_rows(ctx, qtype):
         w.free()
 
 
+def _zero_codes(qtype, blocks):
+    """Blocks whose codes stand for 0 under the scales they have."""
+    if "min_scale" in blocks.dtype.names:
+        blocks["min_scale"] = 0
+    if qtype == qa.Q6_K:
+        blocks["low_bits"] = 0
+        blocks["high_bits"] = 0xAA
+        return
+    blocks["values"] = 8 if qtype == qa.Q4_0 else 0
+    if qtype == qa.Q5_K:
+        blocks["high_bits"] = 0
+
+
+def _raised_activations(qtype, k, n, every, seed):
+    """Weights [k, n] of which every `every`-th row's codes stand for 0, their
+    f64 values, and those rows' numbers: activations there add nothing."""
+    blocks = po.make_weights(qtype, n, k, seed=seed, outliers=qtype >= qa.Q4_K).reshape(k, -1)
+    rows = np.arange(37, k, every)
+    zero = blocks[rows].copy()
+    _zero_codes(qtype, zero)
+    blocks[rows] = zero
+    blocks = blocks.reshape(-1)
+    w = po.dequantize(qtype, blocks).reshape(k, n).astype(np.float64)
+    assert not w[rows].any()
+    return blocks, w, rows
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_row_major_gemv_raised_activations(ctx, qtype, m):
+    """Activations up to 1e20 times the others, at weights that are 0: they add
+    nothing, so the outputs keep the 2-norm error that exact products summed in
+    f32 leave (2e-7: a chunk's sums round to 24 bits, 16 chunks are added)."""
+    k, n = 1040, 512
+    blocks, d, rows = _raised_activations(qtype, k, n, 60, 2400 + qtype)
+    w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+    x0 = po.fill_normal(3400 + m, m * k).reshape(m, k)
+    for ratio in (1.0, 1e4, 1e6, 1e9, 1e20, 1e-20):
+        x = x0.copy()
+        x[:, rows] *= np.float32(ratio)
+        e = x.astype(np.float64) @ d
+        rel = np.linalg.norm(w.linear(x, qa.MODE_F32) - e) / np.linalg.norm(e)
+        assert rel <= 2e-7, (ratio, rel)
+    w.free()
+
+
 @pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
 def test_row_major_gemm_tiles(ctx, qtype):
     """The row-major GEMM at the edges of its tiles: less than one 32-row stage
