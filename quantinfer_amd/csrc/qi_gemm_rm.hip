@@ -17,12 +17,19 @@
 // under 2^15 and held as two f16 halves, 23 bits. v_mfma_f32_16x16x32_f16 then
 // sums the exact products of all parts, smallest first (without that of the two
 // low parts, 2^-22 of the product, 4 x 256 missed the 1e-5 bar), and each 64 k
-// join the running sum in one f32 fused
-// multiply-add with the scale. Error against 64-bit sums, 2-norm, N(0, 1)
-// activations, before (f32 matrix cores) -> now: Q8_0 4096 x 4096 130 rows
-// 1.4e-7 -> 1.2e-7, Q4_K 4096 x 14336 512 rows 2.3e-7 -> 1.8e-7, Q6_K 14336 x
-// 4096 16 rows 1.6e-7 -> 1.4e-7. One-hot activations give the dequantized
-// weights bit for bit, as before.
+// join the running sum in one f32 fused multiply-add with the scale. The low
+// half ends at f16's last bit, 2^-39 of the largest: where a wavefront finds an
+// activation under 2^-18 of its row's largest, what the halves leave makes two
+// further pieces, and the row tiles concerned run a product with each
+// (multiply_rest). So every activation keeps 22 bits down to 2^-53 of the
+// largest of its 64 k; without them, outputs with zero codes at an activation
+// 1e8 times the others had errors of 3e-5 to 6e-5, now as without it, to 1e15
+// times. N(0, 1) activations need them in 4% of a 64-row tile's chunks: 2-3% of
+// the time, finding them 2%.
+// Error against 64-bit sums, 2-norm, N(0, 1) activations, before (f32 matrix
+// cores) -> now: Q8_0 4096 x 4096 130 rows 1.4e-7 -> 1.2e-7, Q4_K 4096 x 14336
+// 512 rows 2.3e-7 -> 1.8e-7, Q6_K 14336 x 4096 16 rows 1.6e-7 -> 1.4e-7. One-hot
+// activations give the dequantized weights bit for bit, as before.
 //
 // Tiling. A workgroup of 4 wavefronts takes one unit (256 outputs), 16 TM rows
 // and one K part; wavefront w its outputs 64 w .. + 63. A stage is 32 weight
@@ -39,9 +46,10 @@
 // 38 matrix instructions of 16 cycles), which slow down from 5 to 8-11 cycles
 // each while the other wavefront of a SIMD runs matrix instructions. MI355X, us
 // per call, the f32 matrix-core kernel (wide scales still take it) -> this one:
-// Q8_0 4096 x 4096 5 rows 15.7 -> 13.2, 16 16.8 -> 14.4, 64 32.9 ->
-// 26.2, 130 65.2 -> 40.4, 512 170 -> 94; Q4_K 4096 x 14336 16 rows 36.8 -> 28.0,
-// 130 235 -> 99, 512 655 -> 299; Q4_0 4096 x 12288 2048 rows 1911 -> 765.
+// Q8_0 4096 x 4096 5 rows 16.3 -> 14.8, 16 17.0 -> 15.6, 130 65.4 -> 42, 512 170
+// -> 93; Q4_K 4096 x 14336 16 rows 38 -> 29.3, 130 235 -> 102, 512 655 -> 316;
+// Q6_K 14336 x 4096 512 rows 619 -> 278; Q4_0 4096 x 12288 64 rows 79 -> 50.5, 512
+// rows 504 -> 283.
 #include "qi_device.h"
 #include "qi_half.h"
 #include "qi_internal.h"
@@ -80,8 +88,10 @@ struct RmLds {
   static constexpr uint32_t kX = kOff + (F::kK45 ? 3 * kRStage * 32 : 0);
   static constexpr uint32_t kXHalf = 2 * TM * 1024;                  // one half [stage][row tile][lane] x 16 B
   static constexpr uint32_t kXP = kX + 2 * kXHalf;                   // x's bf16 pieces, likewise (K45)
-  static constexpr uint32_t kUnsc = kXP + (F::kK45 ? 3 * kXHalf : 0);
-  static constexpr uint32_t kBytes = kUnsc + TM * 16 * 4;
+  static constexpr uint32_t kXRest = kXP + (F::kK45 ? 3 * kXHalf : 0);  // what the halves leave: two pieces, likewise
+  static constexpr uint32_t kUnsc = kXRest + 2 * kXHalf;
+  static constexpr uint32_t kFlag = kUnsc + TM * 16 * 4;             // [row tile][wavefront]: chunk + 1 with a rest
+  static constexpr uint32_t kBytes = kFlag + TM * 4 * 4;
   static_assert(2 * kBytes <= 160 * 1024, "two workgroups on a compute unit");
 };
 
@@ -219,11 +229,13 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
       const uint32_t e = tid + 256 * i, row = e / 16, q = e % 16;
       const bool live = chunk * kRChunk + 4 * q < K;
       float xv[4], v4[4], mx = 0.0f;
+      uint32_t least = ~0u;  // bits of the smallest magnitude above zero, doubled, less 1
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         xv[j] = live ? xr[i][j] : 0.0f;
         v4[j] = F::kD ? xv[j] * f16_bits((j < 2 ? dr[i].x : dr[i].y) >> (16 * (j & 1))) : xv[j];
         mx = fmaxf(mx, fabsf(v4[j]));
+        least = min(least, (__builtin_bit_cast(uint32_t, v4[j]) << 1) - 1);
       }
       mx = fmaxf(mx, dpp_move<0x121>(mx));
       mx = fmaxf(mx, dpp_move<0x122>(mx));
@@ -234,22 +246,56 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
       const int ex = __builtin_isfinite(mx) && mx > 0.0f ? __builtin_amdgcn_frexp_expf(mx) : 0;
       const int sh = min(15 - ex, 125);
       const float scale = __builtin_bit_cast(float, static_cast<uint32_t>(127 + sh) << 23);
+      const float unscale = __builtin_bit_cast(float, static_cast<uint32_t>(127 - sh) << 23);  // 2^-sh
       uint32_t hi[2], lo[2];
+      f32x2 r[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         // both halves rounded to nearest: 23 bits together
         const f32x2 s = {v4[2 * j] * scale, v4[2 * j + 1] * scale};
         const h2 h = __builtin_convertvector(s, h2);
-        const f32x2 r = {s[0] - static_cast<float>(h[0]), s[1] - static_cast<float>(h[1])};
+        r[j] = f32x2{s[0] - static_cast<float>(h[0]), s[1] - static_cast<float>(h[1])};
         hi[j] = h2u(h);
-        lo[j] = h2u(__builtin_convertvector(r, h2));
+        lo[j] = h2u(__builtin_convertvector(r[j], h2));
       }
       const uint32_t at = (q / 8) * TM * 1024 + (row / 16) * 1024 + (16 * (q & 3) + row % 16) * 16 + 8 * ((q >> 2) & 1);
       *reinterpret_cast<uint2*>(lds + L::kX + at) = make_uint2(hi[0], hi[1]);
       *reinterpret_cast<uint2*>(lds + L::kX + L::kXHalf + at) = make_uint2(lo[0], lo[1]);
-      if (q == 0)
-        *reinterpret_cast<float*>(lds + L::kUnsc + 4 * row) =
-            __builtin_bit_cast(float, static_cast<uint32_t>(127 - sh) << 23);  // 2^-sh
+      if (q == 0) *reinterpret_cast<float*>(lds + L::kUnsc + 4 * row) = unscale;
+      // a number under 2^-18 of the row's largest, of which the low half, ending
+      // at f16's last bit, keeps fewer than 22 bits: the rest of this
+      // wavefront's rows, times 2^24, as two halves 2^12 apart. Numbers under
+      // 2^-24 of it go there whole: beside the largest, a matrix instruction
+      // drops bits of products near 2^-42.
+      if (__any(least < (__builtin_bit_cast(uint32_t, unscale * 0x1p-3f) << 1) - 1)) {
+        uint32_t rest[2][2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const h2 l = __builtin_bit_cast(h2, lo[j]);
+          f32x2 t, t2;
+          uint32_t keep = 0;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const float s = v4[2 * j + e] * scale;
+            const bool halves = fabsf(s) >= 0x1p-9f;
+            t[e] = (halves ? r[j][e] - static_cast<float>(l[e]) : s) * 0x1p24f;
+            keep |= halves ? 0xFFFFu << (16 * e) : 0u;
+          }
+          const h2 h = __builtin_convertvector(t, h2);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) t2[e] = (t[e] - static_cast<float>(h[e])) * 0x1p12f;
+          rest[0][j] = h2u(h);
+          rest[1][j] = h2u(__builtin_convertvector(t2, h2));
+          hi[j] &= keep;
+          lo[j] &= keep;
+        }
+        *reinterpret_cast<uint2*>(lds + L::kX + at) = make_uint2(hi[0], hi[1]);
+        *reinterpret_cast<uint2*>(lds + L::kX + L::kXHalf + at) = make_uint2(lo[0], lo[1]);
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          *reinterpret_cast<uint2*>(lds + L::kXRest + p * L::kXHalf + at) = make_uint2(rest[p][0], rest[p][1]);
+        if (lane == 0) *reinterpret_cast<uint32_t*>(lds + L::kFlag + 16 * i + 4 * wave) = chunk + 1;
+      }
       if constexpr (F::kK45) {
         uint32_t p[2][3];
         bf3_pair(xv[0], xv[1], p[0]);
@@ -348,8 +394,40 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
     }
   };
 
+  // a stage's products with what the halves left of the activations, in the
+  // row tiles of the chunk where put_x found such rows (the others' are zero)
+  auto multiply_rest = [&](auto sub, uint32_t chunk) {
+    constexpr int kSub = decltype(sub)::value;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const bool mine = *reinterpret_cast<const uint32_t*>(lds + L::kFlag + 16 * i + 4 * (c >> 2)) == chunk + 1;
+      if (!__any(mine)) continue;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        h8 a = *reinterpret_cast<const h8*>(lds + L::kXRest + p * L::kXHalf + (kSub * TM + i) * 1024 + lane * 16);
+        if (!mine) a = h8{};
+        const float4 us = *reinterpret_cast<const float4*>(lds + L::kUnsc + 4 * (16 * i + 4 * g));
+        const float uu[4] = {us.x, us.y, us.z, us.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v4f s = zero;
+#pragma unroll
+          for (int n = NP - 1; n >= 0; --n)
+            s = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                a, __builtin_bit_cast(h8, read_t(wb + n * kRWPlane + 32 * j, kRWs)), s, 0, 0, 0);
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            acc[i][j][q] = fmaf(uu[q] * (p == 0 ? 0x1p-24f : 0x1p-36f), s[q], acc[i][j][q]);
+          __builtin_amdgcn_sched_barrier(0);  // one tile at a time: its registers are few
+        }
+      }
+    }
+  };
+
   constexpr bool kLate = TM == 4;  // the next chunk's activations a stage later: 256 registers hold no more
   const uint32_t sb = 2 * cb;
+  // a wavefront's flags are its own writes: no barrier before put_x
+  if (lane < static_cast<uint32_t>(TM)) *reinterpret_cast<uint32_t*>(lds + L::kFlag + 16 * lane + 4 * wave) = 0;
   fetch_x(cb);
   fetch_w(sb, wr[0]);
   fetch_w(sb + 1, wr[1]);
@@ -357,15 +435,19 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
     put_x(ch);
     put_w(wr[0]);
     __syncthreads();
+    const bool rest =
+        __any(*reinterpret_cast<const uint32_t*>(lds + L::kFlag + 4 * (lane % (4 * TM))) == ch + 1);
     if constexpr (!kLate) fetch_x(ch + 1);
     fetch_w(2 * ch + 2, wr[0]);
     multiply(std::integral_constant<int, 0>{});
+    if (rest) multiply_rest(std::integral_constant<int, 0>{}, ch);
     __syncthreads();
     put_w(wr[1]);
     __syncthreads();
     if constexpr (kLate) fetch_x(ch + 1);
     fetch_w(2 * ch + 3, wr[1]);
     multiply(std::integral_constant<int, 1>{});
+    if (rest) multiply_rest(std::integral_constant<int, 1>{}, ch);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const float4 us = *reinterpret_cast<const float4*>(lds + L::kUnsc + 4 * (16 * i + 4 * g));

@@ -266,6 +266,27 @@ def test_row_major_gemv_raised_activations(ctx, qtype, m):
 
 
 @pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+@pytest.mark.parametrize("m", [5, 33, 64])
+def test_row_major_gemm_raised_activations(ctx, qtype, m):
+    """The same for the row-major GEMM, every third row raised, up to 1e14
+    times: what the two f16 halves lose there makes further pieces. 2.5e-7: the
+    halves' 23 bits (0.6e-7 of a product's size) beside the f32 sums."""
+    k, n = 1040, 512
+    blocks, d, rows = _raised_activations(qtype, k, n, 60, 2500 + qtype)
+    w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+    x0 = po.fill_normal(3500 + m, m * k).reshape(m, k)
+    for ratio in (1.0, 1e4, 1e5, 1e6, 1e8, 1e11, 1e14, 1e-10):
+        x = x0.copy()
+        x[::3, rows] *= np.float32(ratio)
+        e = x.astype(np.float64) @ d
+        y = w.linear(x, qa.MODE_F32)
+        rel = np.linalg.norm(y - e, axis=1) / np.linalg.norm(e, axis=1)
+        assert rel.max() <= 2.5e-7, (ratio, rel.max())
+        assert w.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+    w.free()
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
 def test_row_major_gemm_tiles(ctx, qtype):
     """The row-major GEMM at the edges of its tiles: less than one 32-row stage
     of k, partial last stages and 64-row chunks, row counts at and past every
