@@ -66,8 +66,8 @@ typedef int32_t qi_hip_status;
  *       Beside an activation far above the others the kernels differ in the
  *       bits that these keep. Row-major: all (1 to 4 rows, and f32 block
  *       scales), 22 bits down to 2^-53 of the largest of the row's 64 k (from
- *       5 rows). Output rows: 2^-30 of the largest of their 256 k (to 8 rows)
- *       or 2^-39 of it (9 rows and more).
+ *       5 rows). Output rows: steps of 2^-29 of the largest of their 32 k (to
+ *       8 rows), of 2^-39 of the largest of their 256 k (9 rows and more).
  * EXACT bit-identical to CpuScalar: per output, acc = acc + x[k]*w[k] in f32,
  *       k ascending, no FMA (backends/cpu/src/matmul.rs:146-157, 319-330).
  * MFMA  f16 operands into f32 matrix-core accumulation (prefill GEMM). */

@@ -2,15 +2,19 @@
 // reference's dense `matmul` (backends/cpu/src/matmul.rs:92-117), y[m, n] =
 // sum_k x[m, k] W[k, n], row-major W, K and N multiples of 4.
 //
-// Arithmetic. Every f32 number is exactly the sum of three bf16 ones: p0 =
-// bf16(v), p1 = bf16(v - p0), p2 = v - p0 - p1 (8 + 8 + 8 bits, no scaling, the
-// whole exponent range). Of the nine products of two such sums the six down
-// to 2^-16 of the largest run on v_mfma_f32_16x16x32_bf16 (the other three are
-// below 2^-24 of it), smallest first from a zero accumulator for each step of
-// 32 k, then one f32 addition to the running sum. Error against 64-bit sums,
+// Arithmetic. Every f32 number times 2^23, the smallest subnormal too, is
+// exactly the sum of three bf16 ones (bf3_pair, qi_half.h: 8 + 8 + 8 bits). Of
+// the nine products of two such sums the six down to 2^-16 of the largest run on
+// v_mfma_f32_16x16x32_bf16 (the other three are below 2^-24 of it), smallest
+// first from a zero accumulator for each step of 32 k, whose sum joins the
+// running one in one f32 fused multiply-add with 2^-46. Numbers from 2^105, or
+// sums of a step from 2^82, overflow: such outputs are recomputed in the
+// reference's order, correct and slow. Error against 64-bit sums,
 // 2-norm, N(0, 1) x N(0, 0.02^2): 1.0e-7 at K = 2048, 1.2e-7 at K = 4096 (300
-// rows); the f32 matrix cores (v_mfma_f32_16x16x4f32, one sixteenth of the
-// bf16 rate, six products here) left 1.8e-7 and 2.3e-7.
+// rows), the same with weights of 2^-126 or activations of 2^-130 (without the
+// factor numbers below 2^-110 lost bits: 1.8e-3 and 3.6e-2 there, for 1-3% less
+// time); the f32 matrix cores (v_mfma_f32_16x16x4f32, one sixteenth of the bf16
+// rate, six products here) left 1.8e-7 and 2.3e-7.
 //
 // Tiling. A workgroup takes 256 columns, 16 TM rows with 4 wavefronts or 32 TM
 // with 8 (two groups that share the stage's weights), and one K part; wavefront
@@ -25,13 +29,14 @@
 // K parts write partial sums that launch_f32w_sum adds in order.
 //
 // What bounds it: the matrix cores from about 128 rows. 2048 x 4096 x 14336
-// runs at 1150 TFLOP/s of bf16 products (192 TFLOP/s of the call's own), the
+// runs at 1107 TFLOP/s of bf16 products (185 TFLOP/s of the call's own), the
 // rate a large bf16 library product reaches here (1105). Below, the weights'
 // conversion and the start of short K parts. MI355X, us per call, the f32
-// matrix-core kernel before -> now: 2048 x 8192, 16 rows 110.4 -> 24.4, 64 97.2
-// -> 36, 128 97.8 -> 45.6, 300 158.1 -> 80, 512 171.3 -> 102; 4096 x 4096, 9
-// rows 216.8 -> 27.0, 300 191.9 -> 87; 4096 x 151936, 64 rows 767 -> 724.
+// matrix-core kernel before -> now: 2048 x 8192, 16 rows 110.4 -> 25.7, 64 97.2
+// -> 36.5, 128 97.8 -> 43.5, 300 158.1 -> 82, 512 171.3 -> 103; 4096 x 4096, 300
+// rows 191.9 -> 85.5.
 #include "qi_device.h"
+#include "qi_half.h"
 #include "qi_internal.h"
 #include "qi_unit.h"
 
@@ -39,9 +44,9 @@ namespace qi {
 
 namespace {
 
+using namespace half;
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
@@ -49,20 +54,6 @@ constexpr uint32_t kBStageK = 32;           // weight rows of a stage: one matri
 constexpr uint32_t kBCols = 256;            // outputs of a workgroup, 64 per wavefront
 constexpr uint32_t kBWs = 2 * kBCols + 32;  // bytes of a weight row in LDS
 constexpr uint32_t kBWPlane = kBStageK * kBWs;
-
-// The pieces of a pair: p[0] + p[1] + p[2] is v exactly, each a bf16 pair.
-__device__ __forceinline__ void bf3_pair(float v0, float v1, uint32_t p[3]) {
-  f32x2 r = {v0, v1};
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-    p[i] = w;
-    if (i < 2) {
-      r[0] -= __builtin_bit_cast(float, w << 16);
-      r[1] -= __builtin_bit_cast(float, w & 0xFFFF0000u);
-    }
-  }
-}
 
 // A wavefront's share of a stage's weights, from memory to three bf16 planes
 // in LDS.
@@ -190,8 +181,6 @@ __global__ __launch_bounds__(256 * WM, 2) void gemm_bf3_kernel(View v, const flo
 #pragma unroll
       for (int p = 0; p < 3; ++p) a[p][i] = *reinterpret_cast<const bf16x8*>(st + xo + p * XPlane + i * 1024);
     read_w(0, b[0]);
-    // pieces of x and w of each product, the smallest first
-    constexpr int kX[6] = {2, 0, 1, 1, 0, 0}, kW[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (j < 3) read_w(j + 1, b[(j + 1) & 1]);
@@ -200,10 +189,12 @@ __global__ __launch_bounds__(256 * WM, 2) void gemm_bf3_kernel(View v, const flo
       for (int q = 0; q < 6; ++q)
 #pragma unroll
         for (int i = 0; i < TM; ++i)
-          sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kX[q]][i], b[j & 1][kW[q]],
+          sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kBf3X[q]][i], b[j & 1][kBf3W[q]],
                                                            q == 0 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : sum[i], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < TM; ++i) acc[i][j] += sum[i];
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(sum[i][q], kBf3Down, acc[i][j][q]);
       beside(j);
     }
   };

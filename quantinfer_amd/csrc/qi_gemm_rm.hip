@@ -63,8 +63,6 @@ namespace {
 
 using namespace half;
 
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
@@ -94,20 +92,6 @@ struct RmLds {
   static constexpr uint32_t kBytes = kFlag + TM * 4 * 4;
   static_assert(2 * kBytes <= 160 * 1024, "two workgroups on a compute unit");
 };
-
-// The pieces of a pair: p[0] + p[1] + p[2] is v exactly, each a bf16 pair.
-__device__ __forceinline__ void bf3_pair(float v0, float v1, uint32_t p[3]) {
-  f32x2 r = {v0, v1};
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
-    p[i] = w;
-    if (i < 2) {
-      r[0] -= __builtin_bit_cast(float, w << 16);
-      r[1] -= __builtin_bit_cast(float, w & 0xFFFF0000u);
-    }
-  }
-}
 
 // The half of a record that one wavefront of a stage converts: of each lane's
 // 64 outputs, the 32 of code chunk `half` (K-quants: steps 2 half, 2 half + 1
@@ -385,11 +369,11 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
           b[p] = __builtin_bit_cast(
               bf16x8, read_t(lds + L::kOff + p * kRStage * 32 + (4 * g + (c >> 2)) * 32 + 8 * (c & 3), 32));
         }
-        constexpr int kX[6] = {2, 0, 1, 1, 0, 0}, kW[6] = {0, 2, 1, 0, 1, 0};
         v4f s = zero;
 #pragma unroll
-        for (int q = 0; q < 6; ++q) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kX[q]], b[kW[q]], s, 0, 0, 0);
-        aoff += s;
+        for (int q = 0; q < 6; ++q) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kBf3X[q]], b[kBf3W[q]], s, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) aoff[q] = fmaf(s[q], kBf3Down, aoff[q]);
       }
     }
   };

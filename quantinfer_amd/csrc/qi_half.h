@@ -13,6 +13,8 @@ namespace half {
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // All-gather across the lane groups: v is V[g] in lane group g; out[g'] = V[g'].
 __device__ __forceinline__ void gather4u(uint32_t u, uint32_t out[4]) {
@@ -320,6 +322,29 @@ __device__ __forceinline__ void split_codes(const typename Unit<QT>::Raw& r, uin
   }
 }
 
+
+// Every f32 number times 2^23 is exactly the sum of three bf16 ones, all normal
+// or zero: p0 = bf16(v), p1 = bf16(v - p0), p2 = v - p0 - p1 for v = 2^23 times
+// the number, 8 + 8 + 8 bits and the last one at or above 2^-126. (Without the
+// factor numbers below 2^-110 end under bf16's last bit, 2^-133.) From 2^105 the
+// first piece is infinite and the sums with it are NaN: their outputs are
+// recomputed in the reference's order.
+constexpr float kBf3Up = 0x1p23f, kBf3Down = 0x1p-46f;  // the factor, and what a sum of products takes back
+__device__ __forceinline__ void bf3_pair(float v0, float v1, uint32_t p[3]) {
+  f32x2 r = {v0 * kBf3Up, v1 * kBf3Up};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+    p[i] = w;
+    if (i < 2) {
+      r[0] -= __builtin_bit_cast(float, w << 16);
+      r[1] -= __builtin_bit_cast(float, w & 0xFFFF0000u);
+    }
+  }
+}
+// The six products of pieces down to 2^-16 of the largest, the smallest first:
+// product q is x's piece kBf3X[q] times w's kBf3W[q].
+constexpr int kBf3X[6] = {2, 0, 1, 1, 0, 0}, kBf3W[6] = {0, 2, 1, 0, 1, 0};
 
 }  // namespace half
 }  // namespace qi

@@ -912,7 +912,7 @@ def test_gguf_upload_same_results(ctx, qtype):
 # ------------------------------------------- F32 weights (the dense matmul)
 #
 # backends/cpu/src/backend.rs:48-60 -> matmul.rs:92-117: W row-major [K, N]
-# f32. F32/AUTO mode: the streaming GEMV up to 16 rows, the f32 matrix-core GEMM above;
+# f32. F32/AUTO mode: the streaming GEMV up to 4 rows, the GEMM on three bf16 pieces a number above;
 # both judged by the F32 bars against CpuScalar's sequential f32 sums and the
 # f64 product.
 
@@ -1000,6 +1000,33 @@ def test_f32_weights_gemm_pieces_are_exact(ctx):
     x[np.arange(m), picks] = 1.0
     assert np.array_equal(wt.linear(x, qa.MODE_F32), w[picks])
     wt.free()
+
+
+def test_f32_weights_gemm_whole_exponent_range(ctx):
+    """One-hot rows give weight rows bit for bit from f32's smallest subnormal
+    to its largest number (from 2^82 by the recompute in the reference's order),
+    at weights of one magnitude per row; and products of small numbers keep the
+    error of the others: 3e-7, as at every magnitude."""
+    k, n = 280, 256
+    rng = np.random.default_rng(9865)
+    exps = np.concatenate([np.arange(-149, -95), [80, 81, 82, 83, 104, 105, 126, 127], np.zeros(k - 62, np.int64)])
+    w = (rng.uniform(1.0, 2.0, (k, n)) * 2.0 ** exps[:, None]).astype(np.float32)
+    w[61] = np.finfo(np.float32).max
+    w[:, ::2] *= -1
+    wt = ctx.weights(qa.F32, qa.ROW_MAJOR, k, n, w)
+    x = np.zeros((62, k), np.float32)
+    x[np.arange(62), np.arange(62)] = 1.0
+    assert np.array_equal(wt.linear(x, qa.MODE_F32), w[:62])
+    wt.free()
+    for wexp, xexp in ((-110, 0), (-120, 0), (0, -115), (0, -125), (30, -130), (60, -60), (-60, 60)):
+        w = po.fill_normal(9866, k * n, 0.02).reshape(k, n) * np.float32(2.0 ** wexp)
+        x = po.fill_normal(9867, 20 * k).reshape(20, k) * np.float32(2.0 ** xexp)
+        wt = ctx.weights(qa.F32, qa.ROW_MAJOR, k, n, w)
+        e = (x.astype(np.float64) @ w.astype(np.float64)) * 2.0 ** -(wexp + xexp)
+        y = wt.linear(x, qa.MODE_F32).astype(np.float64) * 2.0 ** -(wexp + xexp)
+        rel = np.linalg.norm(y - e) / np.linalg.norm(e)
+        assert rel <= 3e-7, (wexp, xexp, rel)
+        wt.free()
 
 
 def test_f32_weights_gemm_under_capture():
