@@ -7,9 +7,11 @@
 // k on the activations' side). A weight is d s (q - z) - b', with d the scale
 // of its (k, 256 outputs) block for the K-quants:
 //   Q4_K/Q5_K  x' = x d; sc (q - z) is an exact f16 integer, z the integer
-//              nearest the window's offset over its scale; the offsets left,
-//              |b'| <= d sc / 2, one per (k, window of 32 outputs), are a
-//              product of their own with x, both as three exact bf16 pieces;
+//              nearest the window's offset over its scale, at most the largest
+//              code; the offsets left, |b'| <= d sc / 2 (more only past the
+//              largest code, where every weight of the window has their sign),
+//              one per (k, window of 32 outputs), are a product of their own
+//              with x, both as three exact bf16 pieces;
 //   Q6_K       x' = x d; sc (q - 32) has up to 12 bits: two exact f16 planes;
 //   Q8_0/Q4_0  x' = x; d q has up to 19 bits: two exact f16 planes (scales in
 //              the range plan_image calls f16_gemm).

@@ -219,6 +219,27 @@ def test_row_major_gemv_rows(ctx, qtype):
         w.free()
 
 
+@pytest.mark.parametrize("qtype", [qa.Q4_K, qa.Q5_K], ids=lambda q: NAMES[q])
+def test_row_major_gemm_offsets_past_the_zero_point(ctx, qtype):
+    """Sub-blocks of scale 0 with a minimum, and minimums past the largest code
+    times the scale (the zero point ends at the largest code): one-hot rows
+    give the dequantized weights to 3 x 2^-24 of each. The offset left past the
+    zero point has the weight's sign and is no larger; it rounds to 24 bits, its
+    sum with the code's product again, and so does the dequantized weight."""
+    k, n = 68, 512
+    rng = np.random.default_rng(2340 + qtype)
+    blocks = po.make_weights(qtype, n, k, seed=2340 + qtype, outliers=True)
+    blocks["scales"] = rng.integers(0, 256, blocks["scales"].shape, dtype=np.uint8)
+    blocks["scales"][::3, :4] &= 0xC0  # scales 0 to 3 of the block: 0
+    blocks["min_scale"] *= np.where(np.arange(blocks.size) % 2, 64, 1).astype(np.float32)
+    w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+    assert w.info().f16_scales == 1
+    y = w.linear(np.eye(k, dtype=np.float32), qa.MODE_F32).astype(np.float64)
+    d = po.dequantize(qtype, blocks).reshape(k, n).astype(np.float64)
+    assert np.all(np.abs(y - d) <= 3 * 2.0 ** -24 * np.abs(d)), np.max(np.abs(y - d) / np.abs(d))
+    w.free()
+
+
 def _zero_codes(qtype, blocks):
     """Blocks whose codes stand for 0 under the scales they have."""
     if "min_scale" in blocks.dtype.names:
