@@ -151,7 +151,12 @@ qi_hip_status qi_hip_linear(qi_hip_ctx *ctx, const qi_hip_weights *w, const floa
 
 /* Same on device buffers, enqueued on `stream` (a hipStream_t; NULL = the
  * context's stream). Returns after the launch; no host synchronisation.
- * x_dev and y_dev must be 16-byte aligned (QI_HIP_INVALID_INPUT otherwise). */
+ * x_dev and y_dev must be 16-byte aligned (QI_HIP_INVALID_INPUT otherwise).
+ * Calls that use a workspace of the context (K-part sums, converted
+ * activations) run one after another, whatever their streams. On a stream
+ * under graph capture nothing is allocated: a call that needs more workspace
+ * than earlier calls left fails, or takes fewer K parts where it can; the
+ * graph holds the workspaces as they are, which a later, larger call frees. */
 qi_hip_status qi_hip_linear_device(qi_hip_ctx *ctx, const qi_hip_weights *w, const float *x_dev,
                                    uint64_t m, float *y_dev, int32_t mode, void *stream);
 

@@ -187,7 +187,7 @@ struct LinearPlan {
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
   uint64_t tail_rows = 0;    // kGemm: last rows that run as a launch of their own with K parts (tail_splits)
   uint32_t tail_splits = 1;
-  uint64_t part_floats = 0;  // kBf3Gemm, kSplitGemm: the most that partial sums may take
+  uint64_t part_floats = 0;  // the GEMMs of plan_parts: the most that partial sums may take
 };
 
 // Rows from which row-major weights (tiled image, K a multiple of 4) take a
@@ -229,21 +229,91 @@ constexpr uint64_t kSplitMinRows = 33;
 // activation records (about 4.1 bytes per activation) stay bounded.
 constexpr uint64_t kSplitChunkRows = 4096;
 
-// K parts of F32 weights' GEMM and of the split-half GEMM, their partial sums
-// within p->part_floats. Calls run in chunks; a shorter last chunk takes its
-// own part count (enqueue_linear asks again).
+// K parts of the F32-accurate GEMMs, their partial sums within p->part_floats.
+// Calls run in chunks; a shorter last chunk takes its own part count
+// (enqueue_linear asks again).
+uint64_t chunk_rows(LinearPlan::Kind kind) {
+  return kind == LinearPlan::kBf3Gemm     ? kBf3ChunkRows
+         : kind == LinearPlan::kSplitGemm ? kSplitChunkRows
+                                          : kRmGemmChunkRows;
+}
+
+uint32_t chunk_parts(const Image& im, const LinearPlan& p, uint64_t rows) {
+  switch (p.kind) {
+    case LinearPlan::kBf3Gemm: return qi::gemm_bf3_plan(im, rows, p.part_floats).parts;
+    case LinearPlan::kRmGemm: return qi::gemm_rm_plan(im, rows, p.part_floats).parts;
+    case LinearPlan::kRowMajorGemm: return qi::rm_gemm_parts(im, rows, p.part_floats);
+    default: return qi::gemm_split_splits(im, rows, p.part_floats);
+  }
+}
+
 void plan_parts(const Image& im, uint64_t m, LinearPlan* p) {
-  const uint64_t rows = p->kind == LinearPlan::kBf3Gemm    ? kBf3ChunkRows
-                        : p->kind == LinearPlan::kRmGemm   ? kRmGemmChunkRows
-                                                           : kSplitChunkRows;
-  const uint64_t chunk = m < rows ? m : rows;
+  const uint64_t rows = chunk_rows(p->kind), chunk = m < rows ? m : rows;
   p->s_floats = 0;
   for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
     if (r == 0) continue;
-    const uint32_t parts = p->kind == LinearPlan::kBf3Gemm  ? qi::gemm_bf3_plan(im, r, p->part_floats).parts
-                           : p->kind == LinearPlan::kRmGemm ? qi::gemm_rm_plan(im, r, p->part_floats).parts
-                                                            : qi::gemm_split_splits(im, r, p->part_floats);
+    const uint32_t parts = chunk_parts(im, *p, r);
     if (parts > 1) p->s_floats = std::max(p->s_floats, static_cast<uint64_t>(parts) * r * im.n);
+  }
+}
+
+// The GEMM of row-major weights, where one takes them.
+bool plan_rm_gemm(const Image& im, uint64_t m, uint64_t part_floats, LinearPlan* p) {
+  const bool f16 = qi::gemm_rm_supported(im);
+  if (!f16 && !qi::rm_gemm_supported(im)) return false;
+  *p = LinearPlan{};
+  p->kind = f16 ? LinearPlan::kRmGemm : LinearPlan::kRowMajorGemm;
+  p->part_floats = part_floats;
+  plan_parts(im, m, p);
+  return true;
+}
+
+// The F32 GEMV in 8-row launches.
+LinearPlan plan_f32_gemv(const Image& im, uint64_t m) {
+  LinearPlan p;
+  p.kind = LinearPlan::kF32Gemv;
+  p.splits = qi::f32w_splits(im);
+  if (p.splits > 1) p.s_floats = static_cast<uint64_t>(p.splits) * (m < 8 ? m : 8) * im.n;
+  return p;
+}
+
+// Row-major workgroups of 32 rows (16 up to 16 rows) fill whole rounds of two
+// per CU without K parts.
+bool rm_fills_chip(const Image& im, uint64_t m) {
+  const uint64_t chunk = m < kRmGemmChunkRows ? m : kRmGemmChunkRows, rest = m % chunk;
+  return qi::rm_gemm_supported(im) && qi::rm_gemm_parts(im, chunk, kRmPartFloats) == 1 &&
+         (rest == 0 || qi::rm_gemm_parts(im, rest, kRmPartFloats) == 1);
+}
+
+// A plan for a stream under capture, which cannot allocate and whose graph
+// outlives the call: K parts as far as their sums fit the workspace that is
+// there (`cap` floats), and none for the calls that fill the chip without, or
+// had no workspace before these GEMMs had parts: a graph of them holds no
+// address that a later, larger call frees.
+void plan_for_capture(const Image& im, uint64_t m, uint64_t cap, LinearPlan* p) {
+  switch (p->kind) {
+    case LinearPlan::kBf3Gemm:
+      // up to 8 rows the GEMV on the workspace that is there: 2048 x 8192 8 rows
+      // 38 us, the GEMM in one part 107
+      if (LinearPlan g = plan_f32_gemv(im, m); m <= 8 && g.s_floats <= cap) *p = g;
+      else p->part_floats = p->s_floats = 0;
+      return;
+    case LinearPlan::kRowMajor:
+      // 3 rows and more can take a GEMM in one part
+      if (m < 3 || im.k % 4 != 0 || (p->s_floats <= cap && !rm_fills_chip(im, m))) return;
+      [[fallthrough]];
+    case LinearPlan::kRmGemm:
+    case LinearPlan::kRowMajorGemm:
+      plan_rm_gemm(im, m, rm_fills_chip(im, m) ? 0 : std::min(cap, kRmPartFloats), p);
+      return;
+    case LinearPlan::kSplitGemm:
+      p->part_floats = std::min(cap, p->part_floats);
+      plan_parts(im, m, p);
+      return;
+    case LinearPlan::kGemm:
+      if (p->s_floats > cap && p->tail_rows > 0) p->tail_rows = p->s_floats = 0;
+      return;
+    default: return;
   }
 }
 
@@ -277,37 +347,18 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     return QI_HIP_OK;
   }
   if (mode != QI_HIP_MODE_EXACT && qi::f32w_gemv_supported(im)) {
-    // F32 weights: the streaming GEMV in 8-row chunks, the matrix-core GEMM above
+    // F32 weights: the GEMM from 5 rows; else (K not a multiple of 4 too) the
+    // streaming GEMV in launches of up to 8 rows
     if (m > qi::kF32GemvMaxRows && qi::gemm_bf3_supported(im)) {
       p->kind = LinearPlan::kBf3Gemm;
       p->part_floats = kBf3PartFloats;
       plan_parts(im, m, p);
       return QI_HIP_OK;
     }
-    p->kind = LinearPlan::kF32Gemv;
-    p->splits = qi::f32w_splits(im);
-    if (p->splits > 1) p->s_floats = static_cast<uint64_t>(p->splits) * (m < 8 ? m : 8) * im.n;
+    *p = plan_f32_gemv(im, m);
     return QI_HIP_OK;
   }
-  if (mode != QI_HIP_MODE_EXACT && qi::gemm_rm_supported(im) && m >= kRmGemmMinRows) {
-    p->kind = LinearPlan::kRmGemm;
-    p->part_floats = kRmPartFloats;
-    plan_parts(im, m, p);
-    return QI_HIP_OK;
-  }
-  if (mode != QI_HIP_MODE_EXACT && qi::rm_gemm_supported(im) && m >= kRmGemmMinRows) {
-    p->kind = LinearPlan::kRowMajorGemm;
-    // chunks of kRmGemmChunkRows rows; a shorter last chunk takes its own
-    // part count (enqueue_linear asks again)
-    const uint64_t chunk = m < kRmGemmChunkRows ? m : kRmGemmChunkRows;
-    for (uint64_t r : {chunk, m > chunk ? m % chunk : 0}) {
-      if (r == 0) continue;
-      const uint32_t parts = qi::rm_gemm_parts(im, r, kRmPartFloats);
-      if (parts > 1) p->s_floats = std::max(p->s_floats, static_cast<uint64_t>(parts) * r * im.n);
-    }
-    p->splits = qi::rm_gemm_parts(im, chunk, kRmPartFloats);
-    return QI_HIP_OK;
-  }
+  if (mode != QI_HIP_MODE_EXACT && m >= kRmGemmMinRows && plan_rm_gemm(im, m, kRmPartFloats, p)) return QI_HIP_OK;
   if (mode != QI_HIP_MODE_EXACT && qi::gemv_rm_supported(im)) {
     p->kind = LinearPlan::kRowMajor;
     const uint32_t rows = qi::gemv_rm_rows(im);
@@ -403,8 +454,7 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
     case LinearPlan::kRowMajorGemm:
       for (uint64_t m0 = 0; m0 < m; m0 += kRmGemmChunkRows) {
         const uint64_t rows = m - m0 < kRmGemmChunkRows ? m - m0 : kRmGemmChunkRows;
-        const uint32_t parts = qi::rm_gemm_parts(im, rows, kRmPartFloats);
-        QI_HIP_TRY(qi::launch_rm_gemm(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, parts, st),
+        QI_HIP_TRY(qi::launch_rm_gemm(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, chunk_parts(im, p, rows), st),
                    "launch row-major GEMM");
       }
       return QI_HIP_OK;
@@ -469,8 +519,7 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
     case LinearPlan::kSplitGemm:
       for (uint64_t m0 = 0; m0 < m; m0 += kSplitChunkRows) {
         const uint64_t rows = m - m0 < kSplitChunkRows ? m - m0 : kSplitChunkRows;
-        const uint32_t sp = qi::gemm_split_splits(im, rows, p.part_floats);
-        QI_HIP_TRY(qi::launch_gemm_split(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, sp,
+        QI_HIP_TRY(qi::launch_gemm_split(im, v, x + m0 * im.k, rows, y + m0 * im.n, sws, chunk_parts(im, p, rows),
                                          reinterpret_cast<uint8_t*>(dws), st),
                    "launch split-half gemm");
       }
@@ -495,15 +544,8 @@ qi_hip_status run_linear(qi_hip_ctx* c, const qi_hip_weights* w, const float* x,
   LinearPlan p;
   qi_hip_status s = plan_linear(w->im, m, mode, &p);
   if (s != QI_HIP_OK) return s;
-  // A stream under capture cannot allocate: fewer K parts where the partial
-  // sums' workspace does not hold them all yet. F32 weights' GEMM, which
-  // needs nothing else from the context, then uses no workspace at all.
-  const bool bf3 = p.kind == LinearPlan::kBf3Gemm;
-  if (p.s_floats > 0 && (bf3 || (p.kind == LinearPlan::kSplitGemm && p.s_floats > c->scap)) && capturing(st)) {
-    p.part_floats = bf3 ? 0 : c->scap;
-    plan_parts(w->im, m, &p);
-  }
-  if (p.tail_rows > 0 && p.s_floats > c->scap && capturing(st)) p.tail_rows = p.s_floats = 0;
+  if (p.s_floats > 0 && (p.part_floats > 0 || p.tail_rows > 0 || p.kind == LinearPlan::kRowMajor) && capturing(st))
+    plan_for_capture(w->im, m, c->scap, &p);
   if ((s = grow_ws(c, st, &c->hbuf, &c->hcap, p.h_floats, "alloc GEMM workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->sbuf, &c->scap, p.s_floats, "alloc split-K workspace")) != QI_HIP_OK) return s;
   if ((s = grow_ws(c, st, &c->dbuf, &c->dcap, p.d_floats, "alloc GEMV workspace")) != QI_HIP_OK) return s;

@@ -1087,6 +1087,67 @@ def test_f32_weights_gemm_under_capture():
         wt.free()
 
 
+def _captured(c, wt, x, n, replays=3):
+    """Outputs of `replays` replays of a captured device call, each after other
+    eager work on the context."""
+    import ctypes
+    from quantinfer_amd import hiprt
+    m = x.shape[0]
+    xd, yd = hiprt.DeviceBuffer.from_array(x), hiprt.DeviceBuffer(m * n * 4)
+    st, h, vp = hiprt.Stream(), hiprt.hip(), ctypes.c_void_p
+    graph, ex = vp(), vp()
+    assert h.hipStreamBeginCapture(vp(st.handle), 1) == 0
+    try:
+        wt.linear_device(xd.ptr, m, yd.ptr, qa.MODE_F32, st.handle)
+    finally:
+        end = h.hipStreamEndCapture(vp(st.handle), ctypes.byref(graph))
+    assert end == 0
+    assert h.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    outs = []
+    for _ in range(replays):
+        yd.zero()
+        hiprt.synchronize()
+        assert h.hipGraphLaunch(ex, vp(st.handle)) == 0
+        st.synchronize()
+        outs.append(yd.to_array(np.float32, (m, n)))
+        wt.linear(x[:1], qa.MODE_F32)
+    h.hipGraphExecDestroy(ex)
+    h.hipGraphDestroy(graph)
+    st.destroy()
+    return outs
+
+
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("qtype,k,n,m", [
+    (qa.Q8_0, 192, 256, 8),     # parts where one ran before the K parts
+    (qa.Q4_K, 2048, 512, 40),   # K parts
+    (qa.Q6_K, 1028, 256, 3),    # the GEMV's K splits
+    (qa.F32, 2048, 512, 7),     # F32 weights: GEMV splits, GEMM parts
+])
+def test_row_major_calls_under_capture(qtype, k, n, m, warm):
+    """A stream under capture allocates nothing: row-major calls of 3 rows and
+    more are captured on a fresh context without K parts, after an eager call
+    with as many as its workspace holds; each replay gives the same outputs,
+    within the F32 bars."""
+    x = po.fill_normal(9881, m * k).reshape(m, k)
+    if qtype == qa.F32:
+        blocks = po.fill_normal(9880, k * n, 0.02).reshape(k, n)
+    else:
+        blocks = po.make_weights(qtype, n, k, seed=9880 + qtype)
+    with qa.Context(0) as c:
+        wt = c.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+        if warm:
+            wt.linear(x, qa.MODE_F32)
+        outs = _captured(c, wt, x, n)
+        if qtype == qa.F32:
+            comp, norm = _f32w_checks(outs[0], x, blocks)
+            assert comp <= F32_TOL and norm <= F32_TOL
+        else:
+            _assert_f32_row_major(outs[0], x, blocks, qtype, n)
+        assert all(o.tobytes() == outs[0].tobytes() for o in outs)
+        wt.free()
+
+
 def test_f32_weights_lm_head_shape(ctx):
     """The unchanged runtime's LM head: [4096, 151936] f32 (a Q6_K head
     dequantized at load, runtime/src/qwen3/loader.rs:47-61), one decode row
