@@ -294,7 +294,7 @@ void plan_for_capture(const Image& im, uint64_t m, uint64_t cap, LinearPlan* p) 
   switch (p->kind) {
     case LinearPlan::kBf3Gemm:
       // up to 8 rows the GEMV on the workspace that is there: 2048 x 8192 8 rows
-      // 38 us, the GEMM in one part 107
+      // 31.7 us in a graph, the GEMM in one part 98 (MI355X)
       if (LinearPlan g = plan_f32_gemv(im, m); m <= 8 && g.s_floats <= cap) *p = g;
       else p->part_floats = p->s_floats = 0;
       return;
@@ -412,16 +412,15 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
 // the plan's size).
 qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const float* x, uint64_t m,
                              float* y, hipStream_t st, float* hws, float* sws, float* dws,
-                             float* silu_act, bool* silu_done) {
+                             float* silu_act) {
   const Image& im = w->im;
   const qi::View v = qi::make_view(im, w->dev);
   switch (p.kind) {
     case LinearPlan::kGemm: {
       qi::GemmArgs ga{v, x, y, m, reinterpret_cast<_Float16*>(hws), p.m_pad};
       ga.splits = p.splits;
-      if (silu_act != nullptr && silu_done != nullptr && ga.splits == 1 && qi::gemm_silu_supported(im)) {
+      if (silu_act != nullptr) {
         ga.act = silu_act;
-        *silu_done = true;
       } else if (p.tail_rows > 0) {
         // whole rounds of workgroups first, then the last rows with K parts
         const uint64_t head = m - p.tail_rows;
@@ -544,6 +543,10 @@ qi_hip_status run_linear(qi_hip_ctx* c, const qi_hip_weights* w, const float* x,
   LinearPlan p;
   qi_hip_status s = plan_linear(w->im, m, mode, &p);
   if (s != QI_HIP_OK) return s;
+  // with the SiLU epilogue one launch takes every row
+  const bool silu = silu_act != nullptr && silu_done != nullptr && p.kind == LinearPlan::kGemm && p.splits == 1 &&
+                    qi::gemm_silu_supported(w->im);
+  if (silu) p.tail_rows = p.s_floats = 0;
   if (p.s_floats > 0 && (p.part_floats > 0 || p.tail_rows > 0 || p.kind == LinearPlan::kRowMajor) && capturing(st))
     plan_for_capture(w->im, m, c->scap, &p);
   if ((s = grow_ws(c, st, &c->hbuf, &c->hcap, p.h_floats, "alloc GEMM workspace")) != QI_HIP_OK) return s;
@@ -551,8 +554,9 @@ qi_hip_status run_linear(qi_hip_ctx* c, const qi_hip_weights* w, const float* x,
   if ((s = grow_ws(c, st, &c->dbuf, &c->dcap, p.d_floats, "alloc GEMV workspace")) != QI_HIP_OK) return s;
   const bool uses_ws = p.h_floats + p.s_floats + p.d_floats > 0;
   if (uses_ws && (s = ws_before(c, st)) != QI_HIP_OK) return s;
-  if ((s = enqueue_linear(w, p, x, m, y, st, c->hbuf, c->sbuf, c->dbuf, silu_act, silu_done)) != QI_HIP_OK)
+  if ((s = enqueue_linear(w, p, x, m, y, st, c->hbuf, c->sbuf, c->dbuf, silu ? silu_act : nullptr)) != QI_HIP_OK)
     return s;
+  if (silu) *silu_done = true;
   return uses_ws ? ws_after(c, st) : QI_HIP_OK;
 }
 
@@ -822,7 +826,7 @@ qi_hip_status qi_hip_linear_device_noalloc(qi_hip_ctx* c, const qi_hip_weights* 
   float* sws = reinterpret_cast<float*>(base + hb);
   float* dws = reinterpret_cast<float*>(base + hb + sb);
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-  return enqueue_linear(w, p, x_dev, m, y_dev, st, hws, sws, dws, nullptr, nullptr);
+  return enqueue_linear(w, p, x_dev, m, y_dev, st, hws, sws, dws, nullptr);
 }
 
 qi_hip_status qi_hip_dequantize_device(qi_hip_ctx* c, const qi_hip_weights* w, float* out_dev,

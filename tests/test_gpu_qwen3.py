@@ -380,3 +380,55 @@ def test_fused_groups_must_share_format(qa, ctx, small):
         m.set_layer(0, layer)
     finally:
         m.free()
+
+
+def test_silu_epilogue_prompt_takes_no_part_sums(qa, ctx):
+    """AUTO mode, 512 prompt rows against 18432 gate|up outputs: 288 row and
+    column blocks, whose last part-filled round would run as a launch with K
+    parts (28 MB of sums) but for the SiLU epilogue, which takes one launch. The
+    other projections (Q6_K) have no parts, so the prompt grows the device's
+    memory by its f16 activations alone (512 x 9216 halves, 9.4 MB)."""
+    import ctypes
+    from quantinfer_amd import hiprt
+    H, I, V = 3072, 9216, 256
+    rng = np.random.default_rng(5)
+
+    def blocks(qtype, k, n):
+        b = np.zeros(k * n // 256, qa.BLOCK_DTYPES[qtype])
+        for f in ("values", "low_bits", "scales"):
+            if f in b.dtype.names:
+                b[f] = rng.integers(0, 16, b[f].shape)
+        b["scale"] = 1e-3
+        return qtype, qa.OUTPUT_ROWS, b
+
+    cfg = small_config(hidden_size=H, intermediate_size=I, num_hidden_layers=1, num_attention_heads=2,
+                       num_key_value_heads=2, head_dim=128, vocab_size=V, max_position_embeddings=1024)
+    with qa.Context(0) as c:
+        m = qa.Qwen3(c, cfg)
+        m.set_embedding(rng.standard_normal((V, H)).astype(np.float32))
+        m.set_layer(0, {
+            "input_layernorm": np.ones(H, np.float32), "post_attention_layernorm": np.ones(H, np.float32),
+            "q_norm": np.ones(128, np.float32), "k_norm": np.ones(128, np.float32),
+            "q_proj": blocks(qa.Q6_K, H, 256), "k_proj": blocks(qa.Q6_K, H, 256), "v_proj": blocks(qa.Q6_K, H, 256),
+            "o_proj": blocks(qa.Q6_K, 256, H), "gate_proj": blocks(qa.Q4_K, H, I), "up_proj": blocks(qa.Q4_K, H, I),
+            "down_proj": blocks(qa.Q6_K, I, H)})
+        m.set_output(np.ones(H, np.float32), blocks(qa.Q6_K, H, V))
+        m.set_mode(qa.MODE_AUTO)
+        cache = m.kv_cache(600)
+        tokens = rng.integers(0, V, 512).astype(np.int32)
+        m.forward(cache, tokens[:130])
+        cache.reset()
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+
+        def free_bytes():
+            hiprt.synchronize()
+            assert hiprt.hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            return free.value
+
+        before = free_bytes()
+        logits, _ = m.forward(cache, tokens)
+        grown = before - free_bytes()
+        assert np.all(np.isfinite(logits))
+        assert grown <= 16 << 20, grown
+        cache.free()
+        m.free()
