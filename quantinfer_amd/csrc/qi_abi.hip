@@ -200,7 +200,7 @@ struct LinearPlan {
 // the f32 GEMM takes 35.1 at 4 rows of Q4_K 4096 x 14336.
 constexpr uint64_t kRmGemmMinRows = 5;
 constexpr uint64_t kRmGemmChunkRows = 4096;
-constexpr uint64_t kRmPartFloats = 8ull << 20;
+using qi::kRmPartFloats;
 
 // F32 weights' GEMM (qi_gemm_bf3.hip): calls run in chunks of kBf3ChunkRows
 // rows; the K parts' partial sums take at most kBf3PartFloats.
@@ -299,8 +299,15 @@ void plan_for_capture(const Image& im, uint64_t m, uint64_t cap, LinearPlan* p) 
       else p->part_floats = p->s_floats = 0;
       return;
     case LinearPlan::kRowMajor:
-      // 3 rows and more can take a GEMM in one part
-      if (m < 3 || im.k % 4 != 0 || (p->s_floats <= cap && !rm_fills_chip(im, m))) return;
+      // 3 rows and more can take a GEMM in one part, fewer the GEMV with its
+      // fewest splits
+      if (m < 3 || im.k % 4 != 0 || (p->s_floats <= cap && !rm_fills_chip(im, m))) {
+        const uint32_t fewest = qi::gemv_rm_fewest_splits(im);
+        if (fewest > 1 && p->s_floats <= cap) return;
+        p->s_floats = fewest > 1 ? p->s_floats / p->splits * fewest : 0;
+        p->splits = fewest;
+        return;
+      }
       [[fallthrough]];
     case LinearPlan::kRmGemm:
     case LinearPlan::kRowMajorGemm:

@@ -852,16 +852,29 @@ bool gemv_rm_supported(const Image& im) {
 
 uint32_t gemv_rm_rows(const Image& im) { return im.tiled ? kRmtRows : 4; }
 
-uint32_t gemv_rm_splits(const Image& im, uint32_t) {
+uint32_t gemv_rm_fewest_splits(const Image& im) {
+  return im.tiled ? static_cast<uint32_t>(((im.tiles + 3) / 4 + 4 * kRmdChunks - 1) / (4 * kRmdChunks))
+                  : gemv_rm_splits(im, 1);
+}
+
+uint32_t gemv_rm_splits(const Image& im, uint32_t rows) {
   const uint32_t be = block_elems(im.qtype);
   if (im.tiled) {
-    // About 512 workgroups (two wavefronts per SIMD on 256 CUs) give each
-    // wavefront one chunk of 64 k, or two at most; then the fewest splits that
-    // keep that.
-    const uint64_t chunks = (im.tiles + 3) / 4, s0 = (512 + im.units - 1) / im.units;
-    const uint64_t per = ((chunks + s0 - 1) / s0 + 3) / 4 <= 1 ? 1 : kRmdChunks;
-    const uint64_t s = (chunks + 4 * per - 1) / (4 * per);
-    return static_cast<uint32_t>(s < 1 ? 1 : s);
+    // One chunk of 64 k for each wavefront, or two. Two workgroups share a
+    // compute unit; time by the workgroups of the busiest of 256 (a pair, and an
+    // odd one at the end), with two chunks 39 a pair and 21 an odd one, with one
+    // 20 and 12: fits to graphs of 17 shapes in every format. MI355X, us per
+    // call, two chunks / one: Q6_K 2048 x 22528 (352 / 704 workgroups) 17.3 / 14.5
+    // (f32 multiply-adds 15.3), 4096 x 10240 (320 / 640) 17.2 / 14.4, 4096 x 14336
+    // (448 / 896) 17.4 / 17.3; Q8_0 4096 x 24576 (768 / 1536) 21.6 / 23.0, 14336 x
+    // 4096 (448 / 896) 16.0 / 17.3.
+    const uint64_t s1 = ((im.tiles + 3) / 4 + 3) / 4, s2 = gemv_rm_fewest_splits(im);
+    auto cost = [&](uint64_t s, uint64_t pair, uint64_t odd) {
+      const uint64_t busiest = (im.units * s + 255) / 256;
+      return busiest / 2 * pair + busiest % 2 * odd;
+    };
+    const bool one = s1 * rows * im.n <= kRmPartFloats && cost(s1, 20, 12) < cost(s2, 39, 21);
+    return static_cast<uint32_t>(one ? s1 : s2);
   }
   // enough K splits for about 1024 workgroups, keeping at least 16 k per
   // wavefront (4 wavefronts per workgroup) and at most 256 splits

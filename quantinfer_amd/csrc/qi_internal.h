@@ -95,11 +95,14 @@ uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t part_floats);
 hipError_t launch_gemm_split(const Image& im, const View& v, const float* x, uint64_t m, float* y, float* part,
                              uint32_t splits, uint8_t* records, hipStream_t st);
 
-// Row-major (blocks along N) GEMV of up to gemv_rm_rows activation rows (4), f32 accumulation, K split over the
-// grid; `part` holds splits * m * n floats when splits > 1.
+// Row-major (blocks along N) GEMV of up to gemv_rm_rows activation rows (4),
+// f32 accumulation, K split over the grid; `part` holds splits * m * n floats
+// when splits > 1.
+constexpr uint64_t kRmPartFloats = 8ull << 20;  // the most that row-major partial sums take where fewer parts do
 bool gemv_rm_supported(const Image& im);
 uint32_t gemv_rm_rows(const Image& im);
 uint32_t gemv_rm_splits(const Image& im, uint32_t m);
+uint32_t gemv_rm_fewest_splits(const Image& im);
 hipError_t launch_gemv_rm(const Image& im, const View& v, const float* x, uint32_t m, float* y, float* part,
                           uint32_t splits, hipStream_t st);
 // Row-major GEMM on a tiled image (K a multiple of 4), any row count: the

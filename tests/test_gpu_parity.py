@@ -240,6 +240,24 @@ def test_row_major_gemm_offsets_past_the_zero_point(ctx, qtype):
     w.free()
 
 
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+def test_row_major_gemv_two_chunks(ctx, qtype):
+    """385 units of 5 chunks of 64 k: one K split, where the first wavefront of
+    a workgroup takes two chunks and the others one (one chunk each would make
+    770 workgroups); the componentwise F32 bar over every output."""
+    k, n = 260, 385 * 256
+    blocks = po.make_weights(qtype, n, k, seed=2330 + qtype)
+    w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+    d = po.dequantize(qtype, blocks).reshape(k, n)
+    for m in (1, 2, 4):
+        x = po.fill_normal(3330 + m, m * k).reshape(m, k)
+        y = w.linear(x, qa.MODE_F32)
+        e = x.astype(np.float64) @ d.astype(np.float64)
+        assert guarded_rel_err(y, e, x, d.T) <= F32_TOL, m
+        assert np.linalg.norm(y - e) <= 2e-7 * np.linalg.norm(e), m
+    w.free()
+
+
 def _zero_codes(qtype, blocks):
     """Blocks whose codes stand for 0 under the scales they have."""
     if "min_scale" in blocks.dtype.names:
@@ -1122,13 +1140,14 @@ def _captured(c, wt, x, n, replays=3):
     (qa.Q8_0, 192, 256, 8),     # parts where one ran before the K parts
     (qa.Q4_K, 2048, 512, 40),   # K parts
     (qa.Q6_K, 1028, 256, 3),    # the GEMV's K splits
+    (qa.Q4_0, 260, 256, 1),     # splits where the fewest are one
     (qa.F32, 2048, 512, 7),     # F32 weights: GEMV splits, GEMM parts
 ])
 def test_row_major_calls_under_capture(qtype, k, n, m, warm):
     """A stream under capture allocates nothing: row-major calls of 3 rows and
-    more are captured on a fresh context without K parts, after an eager call
-    with as many as its workspace holds; each replay gives the same outputs,
-    within the F32 bars."""
+    more, and fewer where one K split can do, are captured on a fresh context
+    without K parts, after an eager call with as many as its workspace holds;
+    each replay gives the same outputs, within the F32 bars."""
     x = po.fill_normal(9881, m * k).reshape(m, k)
     if qtype == qa.F32:
         blocks = po.fill_normal(9880, k * n, 0.02).reshape(k, n)
