@@ -303,7 +303,7 @@ void plan_for_capture(const Image& im, uint64_t m, uint64_t cap, LinearPlan* p) 
       // fewest splits
       if (m < 3 || im.k % 4 != 0 || (p->s_floats <= cap && !rm_fills_chip(im, m))) {
         const uint32_t fewest = qi::gemv_rm_fewest_splits(im);
-        if (fewest > 1 && p->s_floats <= cap) return;
+        if (p->s_floats <= cap && !(fewest == 1 && im.units >= 512)) return;
         p->s_floats = fewest > 1 ? p->s_floats / p->splits * fewest : 0;
         p->splits = fewest;
         return;

@@ -27,8 +27,9 @@
 // transposing reads (ds_read_b64_tr_b8); row strides of 144 bytes keep both
 // sides free of bank conflicts. A workgroup of four wavefronts takes one unit
 // and one K split, each wavefront every fourth chunk of 64 k, at most two, all
-// loaded before the first is used; the wavefronts' sums are added through LDS,
-// the splits by rm_sum_kernel.
+// loaded before the first is used (two wavefronts share a chunk, 128 outputs
+// each, where there are few: gemv_rm_splits); the wavefronts' sums are added
+// through LDS, the splits by rm_sum_kernel.
 // MI355X, us per call (one launch of 1 row, 2-row launches or from 3 rows the
 // f32 GEMM, f32 multiply-adds per code, before -> now): Q4_K 4096 x 14336 1 row
 // 16.1 -> 14.6, 2 27.7 -> 16.0, 4 34.8 -> 21.2; Q5_K 1 row 17.4 -> 16.7; Q6_K
@@ -284,13 +285,15 @@ __device__ __forceinline__ uint64_t rmd_codes(const typename Unit<QT>::Raw& r, u
   }
 }
 
-template <int QT, bool WIDE, int MT, int R>
+template <int QT, bool WIDE, int MT, int C>
 __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* __restrict__ x, uint32_t m,
                                                           uint32_t ksplit, float* __restrict__ out) {
   using U = Unit<QT>;
   using L = RmdLds<QT>;
   constexpr int SW = rmd_subs<QT>(), NT = 2 / SW;  // sub-blocks per lane group and phase, 16-output tiles of each
   constexpr int LV = MT <= 2 ? 2 : 1, Slots = MT * LV;  // levels in one matrix instruction (4 slots of 4 digits)
+  constexpr bool kHalf = C == 0;           // two chunks a workgroup, a phase of one for each wavefront
+  constexpr int R = kHalf ? 1 : C;
   constexpr int SI = MT == 4 ? 1 : SW;  // sub-blocks at a time
   constexpr int X = MT == 4 ? 1 : R;  // chunks of x loaded ahead: 256 registers hold no more
   constexpr bool kOff = window_centered<QT>();
@@ -298,9 +301,9 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t K = static_cast<uint32_t>(v.k), T = v.tiles, C = (T + 3) / 4;
-  const uint32_t cb = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y) * C) / ksplit);
-  const uint32_t ce = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y + 1) * C) / ksplit);
+  const uint32_t K = static_cast<uint32_t>(v.k), T = v.tiles, chunks = (T + 3) / 4;
+  const uint32_t cb = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y) * chunks) / ksplit);
+  const uint32_t ce = static_cast<uint32_t>((static_cast<uint64_t>(blockIdx.y + 1) * chunks) / ksplit);
   const uint8_t* base = v.qs + static_cast<uint64_t>(blockIdx.x) * v.rec.bytes;
   const uint64_t tile_bytes = static_cast<uint64_t>(v.units) * v.rec.bytes;
   uint8_t* const wl = lds + wave * L::kWave;
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
   // records of all of them loaded before the first is used, with no condition
   // (chunks and tiles past the end load the last one again; their activations
   // are zero)
-  const uint32_t c0 = cb + wave, n = c0 < ce ? (ce - c0 + 3) / 4 : 0;
+  const uint32_t c0 = cb + (kHalf ? wave >> 1 : wave), n = c0 < ce ? (ce - c0 + 3) / 4 : 0;
   if (n > 0) {
     typename U::Raw r[R][4];
     float xs[X][4][MT];
@@ -342,6 +345,7 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
       const uint32_t k0 = kRmdChunk * (c0 + 4 * j) + c;  // record t: row k0 + 16 t
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
+        if (kHalf && (wave & 1) != static_cast<uint32_t>(h)) continue;
         // scales of the phase's sub-blocks, their zero points and offsets
         float a[4][SW], b[4][SW];
         uint32_t zt[4];
@@ -523,6 +527,9 @@ hipError_t launch_rmt_rows(const View& v, const float* x, uint32_t m, float* out
     hipLaunchKernelGGL(kern, dim3(v.units, splits), dim3(256), bytes, st, v, x, m, splits, out);
     return hipGetLastError();
   };
+  if constexpr (MT <= 2) {  // at most two chunks a workgroup: two wavefronts for each
+    if ((chunks + splits - 1) / splits <= 2) return go(gemv_rmd_kernel<QT, WIDE, MT, 0>);
+  }
   if (per <= 1) return go(gemv_rmd_kernel<QT, WIDE, MT, 1>);
   if (per <= kRmdChunks) return go(gemv_rmd_kernel<QT, WIDE, MT, kRmdChunks>);
   return hipErrorInvalidValue;
@@ -868,7 +875,13 @@ uint32_t gemv_rm_splits(const Image& im, uint32_t rows) {
     // (f32 multiply-adds 15.3), 4096 x 10240 (320 / 640) 17.2 / 14.4, 4096 x 14336
     // (448 / 896) 17.4 / 17.3; Q8_0 4096 x 24576 (768 / 1536) 21.6 / 23.0, 14336 x
     // 4096 (448 / 896) 16.0 / 17.3.
-    const uint64_t s1 = ((im.tiles + 3) / 4 + 3) / 4, s2 = gemv_rm_fewest_splits(im);
+    const uint64_t chunks = (im.tiles + 3) / 4, s1 = (chunks + 3) / 4, s2 = gemv_rm_fewest_splits(im);
+    // Two wavefronts a chunk where that takes no second workgroup on a compute
+    // unit (1 and 2 rows). A wavefront each / two, 1 row: Q6_K 1024 x 8192 8.3 /
+    // 7.2 (f32 multiply-adds 7.5), 2048 x 2048 8.1 / 7.1 (7.1), Q4_K 512 x 4096
+    // 6.7 / 5.9 (6.4); 512 workgroups, Q4_0 2048 x 8192, 7.2 / 7.2.
+    const uint64_t s0 = (chunks + 1) / 2;
+    if (rows <= 2 && s0 <= 16 && im.units * s0 <= 256) return static_cast<uint32_t>(s0);
     auto cost = [&](uint64_t s, uint64_t pair, uint64_t odd) {
       const uint64_t busiest = (im.units * s + 255) / 256;
       return busiest / 2 * pair + busiest % 2 * odd;
