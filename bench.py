@@ -592,7 +592,7 @@ GEMV_POINTS = ([(0, 1, 4096, 4096, (1,))] +
 # The same points on row-major weights (QuantInfer layout, blocks along N:
 # backends/cpu/src/matmul.rs:14-90), the tiled row-major image: Q4_K at the
 # FFN up shape, Q4_0 at 4096 x 12288, Q8_0 at 4096^2, at their configs' row
-# counts (1 to 4 rows on the row-major GEMV, from 5 the row-major GEMM).
+# counts (1 to 4 rows on the row-major GEMV, from 5 the row-major GEMM at these sizes).
 RM_POINTS = [(2, 3, 4096, 14336, (1, 8)), (1, 2, 4096, 12288, (1, 4, 16)), (0, 1, 4096, 4096, (1,))]
 # the prefill GEMM, Q8_0 and Q4_K, M x (K, N)
 GEMM_POINTS = [(3, q, k, n, (128, 512, 2048)) for q in (1, 3)

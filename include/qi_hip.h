@@ -64,9 +64,9 @@ typedef int32_t qi_hip_status;
  *       split into two f16 halves, weights as exact f16 codes or two f16
  *       halves) accumulated in f32.
  *       Beside an activation far above the others the kernels differ in the
- *       bits that these keep. Row-major: all (1 to 4 rows, and f32 block
- *       scales), 22 bits down to 2^-53 of the largest of the row's 64 k (from
- *       5 rows). Output rows: steps of 2^-29 of the largest of their 32 k (to
+ *       bits that these keep. Row-major: all (1 and 2 rows, 3 and 4 of larger
+ *       weights, f32 block scales), else 22 bits down to 2^-53 of the largest
+ *       of the row's 64 k. Output rows: steps of 2^-29 of the largest of their 32 k (to
  *       8 rows), of 2^-39 of the largest of their 256 k (9 rows and more).
  * EXACT bit-identical to CpuScalar: per output, acc = acc + x[k]*w[k] in f32,
  *       k ascending, no FMA (backends/cpu/src/matmul.rs:146-157, 319-330).

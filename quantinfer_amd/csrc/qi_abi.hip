@@ -187,18 +187,12 @@ struct LinearPlan {
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
   uint64_t tail_rows = 0;    // kGemm: last rows that run as a launch of their own with K parts (tail_splits)
   uint32_t tail_splits = 1;
+  uint32_t launch_rows = 0;  // kRowMajor: rows of a launch
   uint64_t part_floats = 0;  // the GEMMs of plan_parts: the most that partial sums may take
 };
 
-// Rows from which row-major weights (tiled image, K a multiple of 4) take a
-// GEMM instead of the GEMV's launches of up to 4 rows: the f16 matrix-core GEMM
-// (qi_gemm_rm.hip, f16 scales), or where the scales rule it out the f32 one
-// (rm_gemm_kernel). Calls run in chunks of kRmGemmChunkRows rows; partial sums
-// take at most kRmPartFloats. MI355X, us per call, GEMV at 4 rows / f16 GEMM at
-// 5: Q8_0 4096 x 4096 10.7 / 13.2, Q4_K 4096 x 14336 17.5 / 25.9, Q6_K 14336 x
-// 4096 25.7 / 27.5, Q4_0 4096 x 12288 15.7 / 21.0, Q5_K 1024 x 1024 10.0 / 9.1;
-// the f32 GEMM takes 35.1 at 4 rows of Q4_K 4096 x 14336.
-constexpr uint64_t kRmGemmMinRows = 5;
+// Row-major GEMMs run in chunks of kRmGemmChunkRows rows; their partial sums take
+// at most kRmPartFloats.
 constexpr uint64_t kRmGemmChunkRows = 4096;
 using qi::kRmPartFloats;
 
@@ -266,6 +260,21 @@ bool plan_rm_gemm(const Image& im, uint64_t m, uint64_t part_floats, LinearPlan*
   p->part_floats = part_floats;
   plan_parts(im, m, p);
   return true;
+}
+
+// Rows from which row-major weights (tiled image, K a multiple of 4) take a GEMM
+// instead of the GEMV's launches of up to 4 rows: the f16 matrix-core GEMM
+// (qi_gemm_rm.hip, f16 scales), or where the scales rule it out the f32 one
+// (rm_gemm_kernel). MI355X, us per call in a graph, GEMV / f16 GEMM: 4 rows Q8_0
+// 4096 x 4096 11.4 / 13.3, Q4_K 4096 x 14336 21.3 / 27.1, Q4_0 2048 x 8192 10.0 /
+// 10.9; small weights Q4_K 2048 x 2048 9.9 / 8.3, Q8_0 1024 x 8192 10.1 / 9.2, 2
+// rows 7.0 / 8.8; Q6_K, whose two sub-blocks a window double the GEMV's matrix
+// instructions, 3 rows 1024 x 8192 12.7 / 9.4, 4096 x 14336 29.8 / 28.5, 14336 x
+// 4096 31.1 / 28.4, 2 rows 21.9 / 28. GEMV / f32 GEMM at 4 rows: Q4_K 4096 x 14336
+// 21.2 / 34.8, Q6_K 30.6 / 35.2, 1024 x 8192 12.8 / 10.9.
+uint64_t rm_gemm_min_rows(const Image& im) {
+  const bool small = im.k <= 2048 && im.k * im.n <= 1ull << 23, q6 = im.qtype == QI_HIP_Q6_K;
+  return (qi::gemm_rm_supported(im) ? small || q6 : small && q6) ? 3 : 5;
 }
 
 // The F32 GEMV in 8-row launches.
@@ -365,13 +374,20 @@ qi_hip_status plan_linear(const Image& im, uint64_t m, int32_t mode, LinearPlan*
     *p = plan_f32_gemv(im, m);
     return QI_HIP_OK;
   }
-  if (mode != QI_HIP_MODE_EXACT && m >= kRmGemmMinRows && plan_rm_gemm(im, m, kRmPartFloats, p)) return QI_HIP_OK;
+  if (mode != QI_HIP_MODE_EXACT && m >= rm_gemm_min_rows(im) && plan_rm_gemm(im, m, kRmPartFloats, p))
+    return QI_HIP_OK;
   if (mode != QI_HIP_MODE_EXACT && qi::gemv_rm_supported(im)) {
     p->kind = LinearPlan::kRowMajor;
-    const uint32_t rows = qi::gemv_rm_rows(im);
-    const uint32_t chunk = m < rows ? static_cast<uint32_t>(m) : rows;
-    p->splits = qi::gemv_rm_splits(im, chunk);
-    if (p->splits > 1) p->s_floats = static_cast<uint64_t>(p->splits) * chunk * im.n;
+    // sums of 3 and 4 rows past the GEMM's limit (K N above 2^30): the GEMM, or
+    // launches of 2 rows, so that the no-allocation entry point's scratch holds
+    // what it held when these calls had such plans
+    p->launch_rows = qi::gemv_rm_rows(im);
+    for (;; p->launch_rows = 2) {
+      const uint32_t chunk = static_cast<uint32_t>(std::min<uint64_t>(m, p->launch_rows));
+      p->splits = qi::gemv_rm_splits(im, chunk);
+      p->s_floats = p->splits > 1 ? static_cast<uint64_t>(p->splits) * chunk * im.n : 0;
+      if (!im.tiled || chunk <= 2 || p->s_floats <= kRmPartFloats || plan_rm_gemm(im, m, kRmPartFloats, p)) break;
+    }
     return QI_HIP_OK;
   }
   if (mode != QI_HIP_MODE_EXACT && m >= kSplitMinRows && qi::gemm_split_supported(im)) {
@@ -444,9 +460,9 @@ qi_hip_status enqueue_linear(const qi_hip_weights* w, const LinearPlan& p, const
       return QI_HIP_OK;
     }
     case LinearPlan::kRowMajor: {
-      // the blocks-along-N GEMV, gemv_rm_rows rows per launch; a last chunk
+      // the blocks-along-N GEMV, launch_rows rows per launch; a last chunk
       // of fewer rows keeps at most the full chunk's split count
-      const uint32_t per = qi::gemv_rm_rows(im);
+      const uint32_t per = p.launch_rows;
       for (uint64_t m0 = 0; m0 < m; m0 += per) {
         const uint32_t rows = static_cast<uint32_t>(m - m0 < per ? m - m0 : per);
         const uint32_t chunk = m < per ? static_cast<uint32_t>(m) : per;

@@ -1,7 +1,8 @@
 // Row-major (blocks along N) GEMM on the f16 matrix cores with f32 accuracy:
 // y[m, n] = sum_k x[m, k] w(k, n) for QuantInfer-layout weights
 // (backends/cpu/src/backend.rs:62-140 -> matmul.rs:14-90; element values
-// matmul.rs:162-280), 5 rows and more, tiled images with f16 scales.
+// matmul.rs:162-280), from 3 or 5 rows (rm_gemm_min_rows, qi_abi.hip), tiled
+// images with f16 scales.
 //
 // Arithmetic (the split halves of qi_half.h, with the scales that change along
 // k on the activations' side). A weight is d s (q - z) - b', with d the scale

@@ -1,7 +1,8 @@
 // Row-major (blocks along N) GEMV and GEMM, F32 mode: y[m, n] = sum_k x[m, k]
 // w(k, n) for QuantInfer-layout weights (backends/cpu/src/backend.rs:62-140 ->
 // matmul.rs:14-90; element values matmul.rs:162-280). On a tiled image with K
-// a multiple of 4 calls of 5 rows and more take the f16 matrix-core GEMM
+// a multiple of 4 calls of 5 rows and more (Q6_K and small weights: 3, see
+// rm_gemm_min_rows in qi_abi.hip) take the f16 matrix-core GEMM
 // (qi_gemm_rm.hip) or, where the scales are outside its range (f32 block
 // scales), rm_gemm_kernel below: the records dequantized into LDS for the f32
 // matrix cores. Two GEMV kernels by image:

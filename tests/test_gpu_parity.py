@@ -290,8 +290,9 @@ def _raised_activations(qtype, k, n, every, seed):
 def test_row_major_gemv_raised_activations(ctx, qtype, m):
     """Activations up to 1e20 times the others, at weights that are 0: they add
     nothing, so the outputs keep the 2-norm error that exact products summed in
-    f32 leave (2e-7: a chunk's sums round to 24 bits, 16 chunks are added)."""
-    k, n = 1040, 512
+    f32 leave (2e-7: a chunk's sums round to 24 bits, 16 chunks are added). K is
+    no multiple of 4, so that the GEMV takes every row count."""
+    k, n = 1042, 512
     blocks, d, rows = _raised_activations(qtype, k, n, 60, 2400 + qtype)
     w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
     x0 = po.fill_normal(3400 + m, m * k).reshape(m, k)
@@ -322,6 +323,24 @@ def test_row_major_gemm_raised_activations(ctx, qtype, m):
         rel = np.linalg.norm(y - e, axis=1) / np.linalg.norm(e, axis=1)
         assert rel.max() <= 2.5e-7, (ratio, rel.max())
         assert w.linear(x, qa.MODE_F32).tobytes() == y.tobytes()
+    w.free()
+
+
+@pytest.mark.parametrize("qtype", ALL_Q, ids=lambda q: NAMES[q])
+@pytest.mark.parametrize("k,n", [(2048, 4096), (2048, 4352), (2052, 256)])
+def test_row_major_few_rows_either_side(ctx, qtype, k, n):
+    """2 to 5 rows at the sizes where 3 and 4 rows turn from the GEMM to the
+    GEMV (2^23 weights, K = 2048; Q6_K has none): the componentwise F32 bar over
+    every output, and the 2-norm error of f32 sums (2e-7, up to 32 chunks)."""
+    blocks = po.make_weights(qtype, n, k, seed=2320 + qtype, outliers=qtype >= qa.Q4_K)
+    w = ctx.weights(qtype, qa.ROW_MAJOR, k, n, blocks)
+    d = po.dequantize(qtype, blocks).reshape(k, n)
+    for m in (2, 3, 4, 5):
+        x = po.fill_normal(3320 + m, m * k).reshape(m, k)
+        y = w.linear(x, qa.MODE_F32)
+        e = x.astype(np.float64) @ d.astype(np.float64)
+        assert guarded_rel_err(y, e, x, d.T) <= F32_TOL, m
+        assert np.linalg.norm(y - e) <= 2e-7 * np.linalg.norm(e), m
     w.free()
 
 
@@ -1139,7 +1158,8 @@ def _captured(c, wt, x, n, replays=3):
 @pytest.mark.parametrize("qtype,k,n,m", [
     (qa.Q8_0, 192, 256, 8),     # parts where one ran before the K parts
     (qa.Q4_K, 2048, 512, 40),   # K parts
-    (qa.Q6_K, 1028, 256, 3),    # the GEMV's K splits
+    (qa.Q6_K, 1028, 256, 3),    # K parts at 3 rows
+    (qa.Q4_K, 2052, 256, 3),    # the GEMV's K splits, which the GEMM replaces
     (qa.Q4_0, 260, 256, 1),     # splits where the fewest are one
     (qa.F32, 2048, 512, 7),     # F32 weights: GEMV splits, GEMM parts
 ])
