@@ -930,6 +930,30 @@ def e2e_cpu_baseline(cfg, layer: dict, head_blocks) -> dict:
                       f"CpuScalar (matmul.rs:282-332, :92-117), 1 pinned core of {host_cpu()}"}
 
 
+# What an embedded object repeats from the line around it, or only explains.
+_REPEATED = ("n_gpus", "steps", "warmup", "higher_is_better", "scaling", "vs_baseline", "data", "note", "device", "sample",
+             "kind", "cores")
+
+
+def _without(value, keys):
+    if isinstance(value, dict):
+        return {k: _without(v, keys) for k, v in value.items() if k not in keys}
+    return value
+
+
+def short_line(line: dict) -> dict:
+    """The printed line: `line` with its embedded objects free of what they
+    repeat and the configs table as rows, a few KB that a log's tail holds
+    (--full prints `line` itself, about 37 KB). configs rows: config, qtype, m,
+    k, n, us, fraction of the roofline."""
+    out = {k: _without(v, _REPEATED) if k in ("gemv_q8_0", "f32_matmul_head", "gemm", "gemm_f32", "e2e") else v
+           for k, v in line.items()}
+    if "configs" in line:
+        out["configs"] = {kind: [[e["config"], e["qtype"], e["m"], e["k"], e["n"], e["us"], e["roofline"]["frac"]]
+                                 for e in line["configs"][kind]] for kind in ("gemv", "gemv_row_major", "gemm")}
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -955,6 +979,8 @@ def main():
     ap.add_argument("--no-f32head", action="store_true", help="gemv: leave out the F32 LM-head object")
     ap.add_argument("--no-configs", action="store_true",
                     help="gemv: leave out the table of every BASELINE config point")
+    ap.add_argument("--full", action="store_true",
+                    help="gemv: print every field of the embedded objects and of the configs table")
     ap.add_argument("--cpu-simd", action="store_true",
                     help="only the CPU table: scalar and cpu-simd Q8_0/Q4_0 kernels, one core")
     ap.add_argument("--qtype", default="q4_k", help="gemv/gemm: q8_0, q4_0, q4_k, q5_k or q6_k")
@@ -1038,7 +1064,7 @@ def main():
             line["configs"] = configs_table(min(args.steps, 10), min(args.warmup, 3), not args.no_cpu)
         if not args.no_e2e:
             line["e2e"] = e2e_bench(with_cpu=not args.no_cpu)
-    print(json.dumps(line))
+    print(json.dumps(line if args.full else short_line(line), separators=(",", ":")))
 
 
 if __name__ == "__main__":
