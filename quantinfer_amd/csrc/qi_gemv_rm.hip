@@ -573,7 +573,9 @@ hipError_t launch_rm_q(const View& v, const float* x, uint32_t m, float* y, floa
 
 namespace {
 
-// Row-major GEMM, 2 rows and more: y[m, n] = sum_k x[m, k] w(k, n) with the
+// Row-major GEMM of images that the f16 one (qi_gemm_rm.hip) leaves, f32 block
+// scales and Q8_0 / Q4_0 scales outside f16's range, from 3 or 5 rows
+// (rm_gemm_min_rows, qi_abi.hip): y[m, n] = sum_k x[m, k] w(k, n) with the
 // weights dequantized in LDS, never stored to HBM. Workgroup (u, mb, z) takes
 // unit u (outputs 256u .. 256u + 255), rows 16 TM mb .. of x and K part z
 // (tiles [z T / P, (z + 1) T / P)). A stage is 64 weight rows: wavefront w
@@ -586,8 +588,8 @@ namespace {
 // next stage's record and activations are loaded into registers while the
 // matrix cores (v_mfma_f32_16x16x4f32, f32 products) take the current one:
 // wavefront w owns outputs 64w .. 64w + 63 for all 16 TM rows. Each 32-row
-// half of a stage is summed apart and then added to the running sums (the
-// f32 matrix-core GEMM's staged order). One part stores y, recomputing a
+// half of a stage is summed apart and then added to the running sums (one
+// chain over K missed the 1e-5 bar at K = 4096). One part stores y, recomputing a
 // non-finite sum in the reference's order; more store partial sums, which
 // rm_sum_kernel adds in part order.
 constexpr uint32_t kRmgStageK = 64;       // weight rows per stage: one record per wavefront
@@ -842,12 +844,10 @@ hipError_t launch_rm_gemm(const Image& im, const View& v, const float* x, uint64
                          : launch_rm_gemm_q<kQ8_0, false>(v, x, mm, y, part, parts, st);
     case kQ4_0: return w ? launch_rm_gemm_q<kQ4_0, true>(v, x, mm, y, part, parts, st)
                          : launch_rm_gemm_q<kQ4_0, false>(v, x, mm, y, part, parts, st);
-    case kQ4_K: return w ? launch_rm_gemm_q<kQ4_K, true>(v, x, mm, y, part, parts, st)
-                         : launch_rm_gemm_q<kQ4_K, false>(v, x, mm, y, part, parts, st);
-    case kQ5_K: return w ? launch_rm_gemm_q<kQ5_K, true>(v, x, mm, y, part, parts, st)
-                         : launch_rm_gemm_q<kQ5_K, false>(v, x, mm, y, part, parts, st);
-    case kQ6_K: return w ? launch_rm_gemm_q<kQ6_K, true>(v, x, mm, y, part, parts, st)
-                         : launch_rm_gemm_q<kQ6_K, false>(v, x, mm, y, part, parts, st);
+    // K-quants with f16 scales always take the f16 GEMM (gemm_rm_supported)
+    case kQ4_K: return w ? launch_rm_gemm_q<kQ4_K, true>(v, x, mm, y, part, parts, st) : hipErrorInvalidValue;
+    case kQ5_K: return w ? launch_rm_gemm_q<kQ5_K, true>(v, x, mm, y, part, parts, st) : hipErrorInvalidValue;
+    case kQ6_K: return w ? launch_rm_gemm_q<kQ6_K, true>(v, x, mm, y, part, parts, st) : hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
 }

@@ -105,8 +105,8 @@ uint32_t gemv_rm_splits(const Image& im, uint32_t m);
 uint32_t gemv_rm_fewest_splits(const Image& im);
 hipError_t launch_gemv_rm(const Image& im, const View& v, const float* x, uint32_t m, float* y, float* part,
                           uint32_t splits, hipStream_t st);
-// Row-major GEMM on a tiled image (K a multiple of 4), any row count: the
-// weights dequantized into LDS for f32 matrix-core products, K split into
+// Row-major GEMM on a tiled image (K a multiple of 4; launch_rm_gemm: f32 block
+// scales, or Q8_0 / Q4_0), any row count: the weights dequantized into LDS for f32 matrix-core products, K split into
 // `parts` (partial sums in `part`, parts * m * n floats, when parts > 1),
 // non-finite outputs recomputed in the reference's order.
 bool rm_gemm_supported(const Image& im);
