@@ -181,7 +181,8 @@ qi_hip_status grow_ws(qi_hip_ctx* c, hipStream_t st, float** buf, uint64_t* cap,
 // function decides, so that the growing path (run_linear) and the scratch
 // path (qi_hip_linear_device_noalloc) take the same kernels.
 struct LinearPlan {
-  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kRmGemm, kBf3Gemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kExact } kind = kExact;
+  enum Kind { kGemm, kRowMajor, kRowMajorGemm, kRmGemm, kBf3Gemm, kMfma, kSplitGemm, kPlanar, kF32Gemv, kExact };
+  Kind kind = kExact;
   uint64_t m_pad = 0;
   uint32_t splits = 1;  // GEMM K splits, or row-major GEMV K splits per row chunk
   uint64_t h_floats = 0, s_floats = 0, d_floats = 0;  // f16 activations, partials, records
@@ -205,10 +206,13 @@ constexpr uint64_t kBf3PartFloats = 8ull << 20;
 // kernel (qi_gemv_rows.hip) to the split-half kernel (qi_gemv_half.hip): the
 // digit kernel's work grows with the row count (a matrix instruction and a
 // combine per four rows and window), the split-half kernel's does not (all 16
-// rows in one f16 instruction per window half). Measured on MI355X, us per
-// call, digit / split-half: Q4_K 4096x14336 M=2 12.5 / 14.8, M=8 17.7 / 17.1,
-// M=16 29.5 / 23.8; Q4_0 12288x4096 M=4 16.6 / 18.0, M=16 28.1 / 22.9; Q4_K
-// 4096x24576 M=16 49.6 / 38.3.
+// rows in one f16 instruction per window half), but builds its records in a
+// launch of its own. MI355X, us per call, digit / split-half, 8 rows: Q4_K 4096 x
+// 14336 17.0 / 21.2, 14336 x 4096 21.7 / 24.7, 4096 x 4096 11.2 / 16.1, 4096 x
+// 24576 33.3 / 35.1; Q5_K 14336 x 4096 22.1 / 26.6 (5 rows 22.5 / 27.0); Q4_0
+// 4096 x 12288 16.7 / 19.6; Q8_0 4096 x 14336 19.7 / 24.8; Q6_K 14336 x 4096 26.3 /
+// 30.0. 16 rows, when the digit kernel still took them: Q4_K 4096 x 14336 29.5 /
+// 23.8, 4096 x 24576 49.6 / 38.3.
 constexpr uint32_t kHalfMinRows = 9;
 
 // Rows from which output rows take the split-half GEMM (qi_gemm_split.hip)

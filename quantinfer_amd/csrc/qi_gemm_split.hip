@@ -295,9 +295,9 @@ uint32_t gemm_split_splits(const Image& im, uint64_t m, uint64_t part_floats) {
   // (Q6_K 333 x 4096 x 14336) took two rounds of 16 units. Of the counts whose
   // partial sums fit in `part_floats`, the one with the least modelled time:
   // rounds x units of a part x the time of a unit, the sum launch, and the
-  // partial sums' trip through memory. The constants are fits to counts 1 to 16 at 11 shapes (MI355X; model within 10%). Against
-  // the rule before (fill 256 CUs once, rounded up, at least 4 units a part),
-  // us per call: Q4_K M=300 12288 x 4096 136.7 -> 95.4 (80 blocks: 3 parts for
+  // partial sums' trip through memory. The constants are fits to counts 1 to 16
+  // at 11 shapes (MI355X; model within 10%). Against the rule before (fill 256
+  // CUs once, rounded up, at least 4 units a part), us per call: Q4_K M=300 12288 x 4096 136.7 -> 95.4 (80 blocks: 3 parts for
   // 4), 4096 x 6144 82.2 -> 61.4 (2 for 3), 4096 x 4096 63.3 -> 51.3; Q6_K
   // M=333 4096 x 14336 191.2 -> 161.5 (2 for 1); Q4_K M=40 4096 x 4096 32.2 ->
   // 24.5 (16 parts of one unit for 4).
