@@ -310,7 +310,10 @@ Bf3Plan gemm_bf3_plan(const Image& im, uint64_t m, uint64_t max_part_floats) {
   // two (4-wavefront tiles: two fit), for every round of resident workgroups;
   // and with parts the sum launch and the partial sums' trip. The stage times
   // are fits to every tile and part counts 1 to 16 at 2048 x 8192, 16 to 512
-  // rows (MI355X, model mostly within 10%).
+  // rows. Of 17 calls at K 512 to 14336 and N 1024 to 24576 the model is within
+  // 15% at 12 (from 40 rows) and 24% high at 12 us; it is 17-30% low at 16 and 20
+  // rows of large weights, whose bytes, the same for every tile and part count,
+  // it does not count (MI355X).
   struct Tile {
     uint32_t tm, wm;
     double one_us, two_us;
@@ -333,8 +336,8 @@ Bf3Plan gemm_bf3_plan(const Image& im, uint64_t m, uint64_t max_part_floats) {
       const uint64_t n = blocks * p, per = kCUs * (t.wm == 1 ? 2 : 1);
       const uint64_t full = n / per, rest = n % per;
       const double round_us = t.wm == 1 ? t.two_us : t.one_us;
-      const double us = static_cast<double>((stages + p - 1) / p) *
-                            (static_cast<double>(full) * round_us + (rest == 0 ? 0.0 : rest <= kCUs ? t.one_us : t.two_us)) +
+      const double rest_us = rest == 0 ? 0.0 : rest <= kCUs ? t.one_us : t.two_us;
+      const double us = static_cast<double>((stages + p - 1) / p) * (static_cast<double>(full) * round_us + rest_us) +
                         kFixedUs + (p > 1 ? kSumUs + static_cast<double>(bytes) * kPartUsPerByte : 0.0);
       if (best.tm == 0 || us < best_us) {
         best = Bf3Plan{t.tm, t.wm, p};

@@ -354,12 +354,15 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
         part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[i], b[NP - 1], kSub == 0 ? zero : part[i][j], 0, 0, 0);
       if constexpr (NP == 2) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[i], b[0], part[i][j], 0, 0, 0);
+        for (int i = 0; i < TM; ++i)
+          part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[i], b[0], part[i][j], 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[i], b[NP - 1], part[i][j], 0, 0, 0);
+        for (int i = 0; i < TM; ++i)
+          part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[i], b[NP - 1], part[i][j], 0, 0, 0);
       }
 #pragma unroll
-      for (int i = 0; i < TM; ++i) part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[i], b[0], part[i][j], 0, 0, 0);
+      for (int i = 0; i < TM; ++i)
+        part[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[i], b[0], part[i][j], 0, 0, 0);
     }
     if constexpr (F::kK45) {
       // offsets of row tile `wave`: x's pieces times the offsets', eight

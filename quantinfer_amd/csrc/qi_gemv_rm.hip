@@ -261,7 +261,8 @@ struct RmdLds {
 
 __device__ __forceinline__ uint32_t rmd_max(uint32_t v) {
   auto step = [&](auto ctrl) {
-    const uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), decltype(ctrl)::value, 0xF, 0xF, false));
+    const int moved = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), decltype(ctrl)::value, 0xF, 0xF, false);
+    const uint32_t o = static_cast<uint32_t>(moved);
     v = o > v ? o : v;
   };
   step(std::integral_constant<int, 0x121>{});
@@ -462,15 +463,17 @@ __global__ __launch_bounds__(256, 2) void gemv_rmd_kernel(View v, const float* _
             for (int w = 0; w < 4; ++w)
 #pragma unroll
               for (int i = 0; i < SI; ++i) {
-                const i32x4 av = tr(wl + kRmdCodes + (w * SI + i) * L::kDig + (8 * g + (c >> 1)) * 16 + 8 * (c & 1), 16);
+                const uint32_t at = (8 * g + (c >> 1)) * 16 + 8 * (c & 1);
+                const i32x4 av = tr(wl + kRmdCodes + (w * SI + i) * L::kDig + at, 16);
                 const float2 f = *reinterpret_cast<const float2*>(wl + L::kFac + ((w * SI + i) * 4 + g) * 8);
 #pragma unroll
                 for (int q = 0; q < NT; ++q) {
                   const int tile = SW == 2 ? i0 + i : q;
                   const i32x4 bv = tr(wl + (8 * g + (c >> 1)) * kRmdWs + 32 * w + 16 * tile + 8 * (c & 1), kRmdWs);
-                  // lane 16 g + c: the four digit sums of row g, output c of the tile
+                  // lane 16 g + c: the four digit sums of slot g, output c of the tile
                   const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, i32x4{0, 0, 0, 0}, 0, 0, 0);
-                  const float comb = fmaf(static_cast<float>(d[2] + 256 * d[3]), 65536.0f, static_cast<float>(d[0] + 256 * d[1]));
+                  const float low = static_cast<float>(d[0] + 256 * d[1]), high = static_cast<float>(d[2] + 256 * d[3]);
+                  const float comb = fmaf(high, 65536.0f, low);
                   acc[h][w][tile] += kOff ? fmaf(comb, f.x, -f.y) : comb * f.x;
                 }
               }
