@@ -24,12 +24,12 @@
 // half ends at f16's last bit, 2^-39 of the largest: where a wavefront finds an
 // activation under 2^-18 of its row's largest, what the halves leave makes two
 // further pieces, and the row tiles concerned run a product with each
-// (multiply_rest). So every activation keeps 22 bits down to 2^-53 of the
+// (multiply_rest; the second one only where an activation is under 2^-24). So every activation keeps 22 bits down to 2^-53 of the
 // largest of its 64 k; without them, outputs with zero codes at an activation
 // 1e8 times the others had errors of 3e-5 to 6e-5, now as without it, to 1e15
 // times. (x d below 2^-126, x near 2^-113, has the bits of f32's subnormals.)
-// N(0, 1) activations need them in 4% of a 64-row tile's chunks: 2-3% of
-// the time, finding them 2%.
+// N(0, 1) activations need the first in 4% of a 64-row tile's chunks: 1-2%
+// of the time, finding them 2%.
 // Error against 64-bit sums, 2-norm, N(0, 1) activations, before (f32 matrix
 // cores) -> now: Q8_0 4096 x 4096 130 rows 1.4e-7 -> 1.2e-7, Q4_K 4096 x 14336
 // 512 rows 2.3e-7 -> 1.8e-7, Q6_K 14336 x 4096 16 rows 1.6e-7 -> 1.4e-7. One-hot
@@ -51,8 +51,8 @@
 // each while the other wavefront of a SIMD runs matrix instructions. MI355X, us
 // per call, the f32 matrix-core kernel (wide scales still take it) -> this one:
 // Q8_0 4096 x 4096 5 rows 16.3 -> 14.8, 16 17.0 -> 15.6, 130 65.4 -> 42, 512 170
-// -> 93; Q4_K 4096 x 14336 16 rows 38 -> 29.3, 130 235 -> 102, 512 655 -> 316;
-// Q6_K 14336 x 4096 512 rows 619 -> 278; Q4_0 4096 x 12288 64 rows 79 -> 50.5, 512
+// -> 92; Q4_K 4096 x 14336 16 rows 38 -> 29.3, 130 235 -> 102, 512 655 -> 314;
+// Q6_K 14336 x 4096 512 rows 619 -> 272; Q4_0 4096 x 12288 64 rows 79 -> 50.5, 512
 // rows 504 -> 283.
 #include "qi_device.h"
 #include "qi_half.h"
@@ -92,7 +92,7 @@ struct RmLds {
   static constexpr uint32_t kXP = kX + 2 * kXHalf;                   // x's bf16 pieces, likewise (K45)
   static constexpr uint32_t kXRest = kXP + (F::kK45 ? 3 * kXHalf : 0);  // what the halves leave: two pieces, likewise
   static constexpr uint32_t kUnsc = kXRest + 2 * kXHalf;
-  static constexpr uint32_t kFlag = kUnsc + TM * 16 * 4;             // [row tile][wavefront]: chunk + 1 with a rest
+  static constexpr uint32_t kFlag = kUnsc + TM * 16 * 4;             // [row tile][wavefront]: 2 (chunk + 1) + second piece
   static constexpr uint32_t kBytes = kFlag + TM * 4 * 4;
   static_assert(2 * kBytes <= 160 * 1024, "two workgroups on a compute unit");
 };
@@ -255,7 +255,8 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
       // wavefront's rows, times 2^24, as two halves 2^12 apart. Numbers under
       // 2^-24 of it go there whole: beside the largest, a matrix instruction
       // drops bits of products near 2^-42.
-      if (__any(least < (__builtin_bit_cast(uint32_t, unscale * 0x1p-3f) << 1) - 1)) {
+      auto under = [&](float bound) { return __any(least < (__builtin_bit_cast(uint32_t, unscale * bound) << 1) - 1); };
+      if (under(0x1p-3f)) {
         uint32_t rest[2][2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -282,7 +283,8 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
 #pragma unroll
         for (int p = 0; p < 2; ++p)
           *reinterpret_cast<uint2*>(lds + L::kXRest + p * L::kXHalf + at) = make_uint2(rest[p][0], rest[p][1]);
-        if (lane == 0) *reinterpret_cast<uint32_t*>(lds + L::kFlag + 16 * i + 4 * wave) = chunk + 1;
+        const uint32_t second = under(0x1p-9f) ? 1 : 0;  // numbers above it end with the first piece
+        if (lane == 0) *reinterpret_cast<uint32_t*>(lds + L::kFlag + 16 * i + 4 * wave) = 2 * (chunk + 1) + second;
       }
       if constexpr (F::kK45) {
         uint32_t p[2][3];
@@ -391,10 +393,13 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
     constexpr int kSub = decltype(sub)::value;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const bool mine = *reinterpret_cast<const uint32_t*>(lds + L::kFlag + 16 * i + 4 * (c >> 2)) == chunk + 1;
+      const uint32_t flag = *reinterpret_cast<const uint32_t*>(lds + L::kFlag + 16 * i + 4 * (c >> 2));
+      const bool mine = flag / 2 == chunk + 1;
       if (!__any(mine)) continue;
+      const bool second = __any(mine && flag % 2 != 0);
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
+        if (p == 1 && !second) break;
         h8 a = *reinterpret_cast<const h8*>(lds + L::kXRest + p * L::kXHalf + (kSub * TM + i) * 1024 + lane * 16);
         if (!mine) a = h8{};
         const float4 us = *reinterpret_cast<const float4*>(lds + L::kUnsc + 4 * (16 * i + 4 * g));
@@ -427,7 +432,7 @@ __global__ __launch_bounds__(256, 2) void gemm_rm_kernel(View v, const float* __
     put_w(wr[0]);
     __syncthreads();
     const bool rest =
-        __any(*reinterpret_cast<const uint32_t*>(lds + L::kFlag + 4 * (lane % (4 * TM))) == ch + 1);
+        __any(*reinterpret_cast<const uint32_t*>(lds + L::kFlag + 4 * (lane % (4 * TM))) / 2 == ch + 1);
     if constexpr (!kLate) fetch_x(ch + 1);
     fetch_w(2 * ch + 2, wr[0]);
     multiply(std::integral_constant<int, 0>{});
