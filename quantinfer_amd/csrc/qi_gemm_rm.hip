@@ -24,10 +24,10 @@
 // half ends at f16's last bit, 2^-39 of the largest: where a wavefront finds an
 // activation under 2^-18 of its row's largest, what the halves leave makes two
 // further pieces, and the row tiles concerned run a product with each
-// (multiply_rest; the second one only where an activation is under 2^-24). So every activation keeps 22 bits down to 2^-53 of the
-// largest of its 64 k; without them, outputs with zero codes at an activation
-// 1e8 times the others had errors of 3e-5 to 6e-5, now as without it, to 1e15
-// times. (x d below 2^-126, x near 2^-113, has the bits of f32's subnormals.)
+// (multiply_rest; the second one only where an activation is under 2^-24). So
+// every activation keeps 22 bits down to 2^-53 of the largest of its 64 k;
+// without them, outputs with zero codes at an activation 1e8 times the others
+// had errors of 3e-5 to 6e-5, now as without it, to 1e15 times. (x d below 2^-126, x near 2^-113, has the bits of f32's subnormals.)
 // N(0, 1) activations need the first in 4% of a 64-row tile's chunks: 1-2%
 // of the time, finding them 2%.
 // Error against 64-bit sums, 2-norm, N(0, 1) activations, before (f32 matrix
